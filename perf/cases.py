@@ -40,9 +40,9 @@ def _case(name, kind, problem, n, steps, rk=True, mixed=False, driver="vertical"
 
 def listed():
     return [
-        # smallest 3D run (the smoke test's grid): launches and the latency
-        # of one tile are all there is
-        _case("strat3d_16x12x12", "forward", "stratified", (16, 12, 12), 1),
+        # smallest 3D run (the smoke test's grid), a step from a checkpoint:
+        # launches and the latency of one tile are all there is
+        _case("strat3d_16x12x12", "forward", "stratified", (16, 12, 12), 1, restart=True),
         # 2D Orszag-Tang vortex, periodic, CFL time step, RK4: a short run
         # from a checkpoint
         _case("ot2d_128", "forward", "orszag_tang", (128, 128), 10, driver="none", restart=True),
@@ -94,7 +94,7 @@ def draw(rng):
     n = (around(size, 10), around(size, 10), around(size, 10))
     steps = rng.randint(1, 3) if size > 60 else rng.randint(1, 8)
     driver = rng.choice(["vertical", "torsional", "none"])
-    return _case(None, kind, "stratified", n, steps, rk, mixed, driver, kind == "forward" and not rk)
+    return _case(None, kind, "stratified", n, steps, rk, mixed, driver, kind == "forward" and (not rk or size < 40))
 
 
 # --------------------------------------------------------------------------
