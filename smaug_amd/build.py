@@ -23,6 +23,9 @@ HIPCC_FLAGS = [
     "-ffp-contract=fast",
     # no packed FP32 instructions (they are not used on purpose anywhere)
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the stage kernels read their by-value arguments in several hundred
+    # places; past 300 uses the compiler keeps a copy in scratch memory
+    "-mllvm", "-instcombine-max-copied-from-constant-users=10000",
     "-Wno-unused-value", "-Wno-pass-failed",
 ]
 

@@ -41,23 +41,23 @@ struct Geo {
 };
 
 // evolved-field indices
-__host__ __device__ inline int fRHO() { return 0; }
-__host__ __device__ inline int fMOM(int d) { return 1 + d; }
-__host__ __device__ inline int fE(int nd) { return 1 + nd; }
-__host__ __device__ inline int fB(int nd, int d) { return 2 + nd + d; }
+__host__ __device__ __forceinline__ int fRHO() { return 0; }
+__host__ __device__ __forceinline__ int fMOM(int d) { return 1 + d; }
+__host__ __device__ __forceinline__ int fE(int nd) { return 1 + nd; }
+__host__ __device__ __forceinline__ int fB(int nd, int d) { return 2 + nd + d; }
 // background indices
-__host__ __device__ inline int bEB() { return 0; }
-__host__ __device__ inline int bRHOB() { return 1; }
-__host__ __device__ inline int bBB(int d) { return 2 + d; }
+__host__ __device__ __forceinline__ int bEB() { return 0; }
+__host__ __device__ __forceinline__ int bRHOB() { return 1; }
+__host__ __device__ __forceinline__ int bBB(int d) { return 2 + d; }
 // prim indices
-__host__ __device__ inline int pV(int d) { return d; }
-__host__ __device__ inline int pQE(int nd) { return nd; }
+__host__ __device__ __forceinline__ int pV(int d) { return d; }
+__host__ __device__ __forceinline__ int pQE(int nd) { return nd; }
 
 // Boundary-table indices the reference's gradient calls pass as "field"
 // (quirk Q2: derived and temporary arrays index boundtype[] with their own
 // enum value).  Values of the DEV/TEV enums in include/iotypes.h:225-242.
-__host__ __device__ inline int zFLUX(int nd) { return nd; }  // DEV flux
-__host__ __device__ inline int zVEL(int d) { return d; }     // DEV vel1+d
+__host__ __device__ __forceinline__ int zFLUX(int nd) { return nd; }  // DEV flux
+__host__ __device__ __forceinline__ int zVEL(int d) { return d; }     // DEV vel1+d
 constexpr int zRHO = 0, zTMP1 = 0, zTMP3 = 2, zTMP4 = 3, zTMP5 = 4, zTMP7 = 6, zTMP8 = 7;
 
 // ---------------------------------------------------------------------------
@@ -71,12 +71,12 @@ constexpr int zRHO = 0, zTMP1 = 0, zTMP3 = 2, zTMP4 = 3, zTMP5 = 4, zTMP7 = 6, z
 //   7 asymm     the symm map with the sign flipped    (src/gradops.cu:1325-1466)
 constexpr int BC_PERIODIC = 0, BC_CONT = 3, BC_CONTCD4 = 4, BC_FIXED = 5, BC_SYMM = 6, BC_ASYMM = 7;
 
-__host__ __device__ inline bool bc_is_ghost(int x, int n) { return x < 2 || x > n - 3; }
-__host__ __device__ inline double bc_sign(int type) { return type == BC_ASYMM ? -1.0 : 1.0; }
+__host__ __device__ __forceinline__ bool bc_is_ghost(int x, int n) { return x < 2 || x > n - 3; }
+__host__ __device__ __forceinline__ double bc_sign(int type) { return type == BC_ASYMM ? -1.0 : 1.0; }
 
 // interior coordinate the ghost coordinate x copies (x itself when x is
 // not a ghost, -1 for a fixed ghost)
-__host__ __device__ inline int bc_src(int type, int x, int n, int nd) {
+__host__ __device__ __forceinline__ int bc_src(int type, int x, int n, int nd) {
   if (!bc_is_ghost(x, n)) return x;
   switch (type) {
     case BC_PERIODIC:
@@ -97,7 +97,7 @@ __host__ __device__ inline int bc_src(int type, int x, int n, int nd) {
 // ghost coordinates whose value is copied from interior coordinate y (at
 // most mmax of them; with n >= 8 there are at most two); returns how many
 // were written to out[].  The inverse of bc_src, written out per type.
-__host__ __device__ inline int bc_images(int type, int y, int n, int nd, int* out, int mmax = 4) {
+__host__ __device__ __forceinline__ int bc_images(int type, int y, int n, int nd, int* out, int mmax = 4) {
   int m = 0;
   auto put = [&](int g) {
     if (m < mmax) out[m++] = g;
@@ -136,7 +136,7 @@ __host__ __device__ inline int bc_images(int type, int y, int n, int nd, int* ou
 struct Img2 {
   int m, g0, g1;
 };
-__host__ __device__ inline Img2 bc_images2(int type, int y, int n, int nd) {
+__host__ __device__ __forceinline__ Img2 bc_images2(int type, int y, int n, int nd) {
   if (type == BC_FIXED) return Img2{0, 0, 0};
   if (type == BC_PERIODIC) {
     if (y == n - 4) return Img2{1, 0, 0};
@@ -166,23 +166,23 @@ __host__ __device__ inline Img2 bc_images2(int type, int y, int n, int nd) {
 }
 
 // zeroing of grad3dn at interior cells: first/last two interior layers
-__device__ inline bool z4(const Geo& G, int idx, int d, int x) {
+__device__ __forceinline__ bool z4(const Geo& G, int idx, int d, int x) {
   const int n = G.n[d];
   return ((G.zm[idx] >> d) & 1u) && (x == 2 || x == 3 || x == n - 4 || x == n - 3);
 }
 // zeroing of grad1l3n/grad1r3n/grad13n at cells whose other coordinates
 // are inside 1..n-2: the first and last interior layer
-__device__ inline bool z1(const Geo& G, int idx, int d, int x) {
+__device__ __forceinline__ bool z1(const Geo& G, int idx, int d, int x) {
   return ((G.zm[idx] >> d) & 1u) && (x == 2 || x == G.n[d] - 3);
 }
 // the same tests where the caller knows whether x can lie on a zeroed
 // layer at all (EDGE false: x in [5, n-6], never zeroed)
 template <bool EDGE>
-__device__ inline bool z4e(const Geo& G, int idx, int d, int x) {
+__device__ __forceinline__ bool z4e(const Geo& G, int idx, int d, int x) {
   return EDGE && z4(G, idx, d, x);
 }
 template <bool EDGE>
-__device__ inline bool z1e(const Geo& G, int idx, int d, int x) {
+__device__ __forceinline__ bool z1e(const Geo& G, int idx, int d, int x) {
   return EDGE && z1(G, idx, d, x);
 }
 
@@ -195,7 +195,7 @@ __device__ inline bool z1e(const Geo& G, int idx, int d, int x) {
 // stray value survives at padded cell H iff its writer t = L(H) - C is a
 // valid thread not earlier than H's zeroing thread.  Returns the unpadded
 // linear index of the source cell, or -1 for zero.
-__host__ __device__ inline long long halo_r_src(const Geo& G, const int* pc) {
+__host__ __device__ __forceinline__ long long halo_r_src(const Geo& G, const int* pc) {
   const long long P0 = G.n[0] + 2, P1 = G.n[1] + 2;
   long long LH, C, tz;
   int z0 = pc[0] < G.n[0] - 1 ? pc[0] : G.n[0] - 1;

@@ -1,19 +1,21 @@
 // smaug_rhs.hip -- tiled right-hand side of one SMAUG stage (k_rhs).
 //
-// One workgroup owns a tile of interior cells (8x4x8 in 3D, 16x16 in 2D,
-// 256 threads, one cell each) and builds every term of the reference step
-// for it from LDS-staged data, so each intermediate is computed once:
-//   1. flux phase, per direction d: the eight fluxes F_f^d of the tile
-//      extended by two cells along d go to LDS, then each thread takes the
-//      4th-order divergence (centdiff1/centdiff2).
+// One workgroup owns a tile of interior cells (TileT: 8x4x8 or 8x8x8 in 3D,
+// 16x16 in 2D; one cell or a pair along dim 0 per thread) and builds every
+// term of the reference step for it from LDS-staged data, so each
+// intermediate is computed once:
+//   1. flux phase, per direction d: the fluxes F_f^d of the tile extended by
+//      two cells along d go to LDS, then each thread takes the 4th-order
+//      divergence (centdiff1/centdiff2).
 //   2. hyperdiffusion phase, per variable q (rho, e_int, v_f, b_f): q is
 //      staged as the tile plus a 3-cell halo (with the reference's halo
-//      substitutions of quirks Q7/Q8); for every direction the coefficients
-//      nu_{i+-1/2} and the cross-term products of the off-diagonal momentum
-//      and magnetic sources are formed once per cell of the tile extended by
-//      one cell along the cross direction, then each thread applies the
-//      diagonal and off-diagonal sources.  The v_f phase also applies the
-//      background energy terms, which need gradients of v_f only.
+//      substitutions of quirks Q7/Q8); every direction's window of a cell
+//      gives nu_{i+-1/2}, the diagonal sources and the cross-term products of
+//      the off-diagonal momentum and magnetic sources, which are also formed
+//      on the layer outside the tile along the cross direction; after a
+//      barrier each thread takes the products' differences.  The v_f phase
+//      also applies the background energy terms, which need gradients of v_f
+//      only.
 //   3. gravity, the stage update, the user source, the RK combination and
 //      the ghost-cell images (boundaries fused).
 // The stencils work in the stencil precision SH: FP64 (the state itself),
@@ -22,6 +24,24 @@
 // workgroup and so raises the number resident per CU.  The own-cell values,
 // the background terms, the stage update (base + h*acc), the driver and the
 // RK combination are FP64 in both.
+//
+// What bounds it and how that shaped the code (MI355X):
+//  * a tile's phases are a chain of memory round trips and barriers, so time
+//    falls with every workgroup more that a CU holds: sums are pinned phase
+//    by phase (pin) and loads of the own cell repeated rather than kept, which
+//    took the FP64 kernel from 150 to 109 VGPRs, and its LDS from 52 to 34 KB:
+//    four workgroups per CU instead of three (FP64, k_rhs at 128^3: 0.676 ->
+//    0.513 ms; FP32 0.470 -> 0.403);
+//  * the code of a tile at the grid's edge (masks, halo substitutions, ghost
+//    images) streamed 211 KB of instructions through caches of 64 KB per two
+//    CUs; loops in place of unrolled bodies made it 50 KB (one tile by itself:
+//    73 -> 48 us);
+//  * on grids of few tiles nothing hides a round trip: those keep every box
+//    in LDS at once (ALL: 6 barriers for 20, 48 -> 33 us per tile);
+//  * on large FP64 grids the traffic of the boxes counts: a tile of twice the
+//    cells re-reads a third less halo (k_rhs at 256^3: 4.60 ms before, 3.73
+//    with the small tile, 3.51 with the wide one; 14.9 GB fetched from beyond
+//    L2 at 4.2 TB/s, of 5.0 TB/s that a streaming pass reaches).
 #include <math.h>
 
 #include <type_traits>
@@ -32,708 +52,276 @@
 
 namespace smaug {
 
-template <int ND>
-struct Tile;
-// 3D tile 8 x 4 x 8: dim 0 (contiguous) 8 wide for coalesced rows; the
-// workgroups resident on one XCD cover whole x-rows and neighbouring
-// y-rows, so the tile is deep in z, the direction whose neighbour tiles are
-// least likely to still be in L2 (fewer halo planes re-fetched per cell)
-template <>
-struct Tile<3> {
-  static constexpr int X = 8, Y = 4, Z = 8;
-};
-template <>
-struct Tile<2> {
-  static constexpr int X = 16, Y = 16, Z = 1;
+// Tile of interior cells a workgroup owns: X x Y x Z, XC cells per thread
+// (neighbours along dim 0).
+template <int ND_, int X_, int Y_, int Z_, int XC_>
+struct TileT {
+  static constexpr int ND = ND_, X = X_, Y = Y_, Z = Z_, XC = XC_, NT = X_ * Y_ * Z_ / XC_;
 };
 
-constexpr int imax(int a, int b) { return a > b ? a : b; }
+__host__ __device__ constexpr int imax(int a, int b) { return a > b ? a : b; }
+__host__ __device__ constexpr int imin(int a, int b) { return a < b ? a : b; }
 
-template <int ND>
+template <class TL>
 struct Lay {
-  static constexpr int TX = Tile<ND>::X, TY = Tile<ND>::Y, TZ = Tile<ND>::Z;
+  static constexpr int ND = TL::ND, XC = TL::XC, NT = TL::NT;
+  static constexpr int TX = TL::X, TY = TL::Y, TZ = TL::Z;
   static constexpr int NP = 2 + 2 * ND;
+  // halo widths along dim 0: with two cells per thread each box starts an
+  // even number of cells before the tile, so a thread's pair is aligned
+  static constexpr int HX = XC == 2 ? 4 : 3, RX = XC == 2 ? 2 : 1;
   // q box: tile + 3-cell halo
-  static constexpr int QX = TX + 6, QY = TY + 6, QZ = ND == 3 ? TZ + 6 : 1;
+  static constexpr int QX = TX + 2 * HX, QY = TY + 6, QZ = ND == 3 ? TZ + 6 : 1;
   static constexpr int QN = QX * QY * QZ;
   // region: tile extended by one cell along one axis
-  static constexpr int RN = ND == 3 ? imax(imax((TX + 2) * TY * TZ, TX * (TY + 2) * TZ), TX * TY * (TZ + 2))
-                                    : imax((TX + 2) * TY, TX * (TY + 2));
+  static constexpr int RN = ND == 3 ? imax(imax((TX + 2 * RX) * TY * TZ, TX * (TY + 2) * TZ), TX * TY * (TZ + 2))
+                                    : imax((TX + 2 * RX) * TY, TX * (TY + 2));
   // flux region: tile extended by two cells along one axis
   static constexpr int FN = ND == 3 ? imax(imax((TX + 4) * TY * TZ, TX * (TY + 4) * TZ), TX * TY * (TZ + 4))
                                     : imax((TX + 4) * TY, TX * (TY + 4));
-  static constexpr int HYP = QN + 4 * RN;
-  static constexpr int FLX = NP * FN;
-  // cell box: tile + 1-cell halo; box 0 rho_t, boxes 1..ND the
-  // components of the phase's vector (m in the momentum phases, b in the
-  // field phases); it sits ahead of the area the phases share
-  static constexpr int PX = TX + 2, PY = TY + 2, PZ = ND == 3 ? TZ + 2 : 1;
+  // q box and the ND region arrays of a phase: one product per cross
+  // direction and the sum of their energy products
+  static constexpr int HYP = QN + ND * RN;
+  static constexpr int FLX = (NP - 1) * FN;  // the flux of b_d along d is zero and not kept
+  // rho_t on the tile + 1-cell halo, ahead of the area the phases share
+  static constexpr int PX = TX + 2 * RX, PY = TY + 2, PZ = ND == 3 ? TZ + 2 : 1;
   static constexpr int PN = PX * PY * PZ;
-  static constexpr int CB = (ND + 1) * PN;
-  static constexpr int SHR = HYP > FLX ? HYP : FLX;  // area the phases share
+  static constexpr int SHR = imax(HYP, FLX);  // area the phases share
   // spacing table of a tensor-product grid: delx and 1/delx at the tile's
-  // coordinates along each axis (for the cross-term border cells)
+  // coordinates along each axis
   static constexpr int DXT = TX + TY + TZ;
-  static constexpr int SMEM = CB + SHR + 2 * DXT;
+  static constexpr int DXO = imax(PN + SHR, 2 * QN);  // (the rho and q_e boxes are staged together)
+  static constexpr int SMEM = DXO + 2 * DXT;
+  // the same with every box, every direction's fluxes and the products of a
+  // group of phases at once
+  static constexpr int DXO_ALL = imax(PN + NP * QN + ND * ND * RN, ND * FLX);
+  static constexpr int SMEM_ALL = DXO_ALL + 2 * DXT;
+  static_assert(XC == 1 || (QN % 2 == 0 && RN % 2 == 0 && FN % 2 == 0 && PN % 2 == 0), "pairs stay aligned");
 };
 
-// cell box of the tile plus one cell: rho_t = rho + rho_b (when with_rho)
-// and the ND components f0.. of the state, in the stencil precision SH
-// (cells outside the grid hold 0 and are never read).  Loads and stores are
-// separate steps so the loads can share a round trip with a q box's.
-template <int ND, typename SH>
-struct CellBox {
-  SH* CBX;  // null: no cell box with this q box
-  bool with_rho;
-  int f0;
-  bool shell = false;  // 3D: the tile's own cells are already in the box
-                       // (written from the flux phase's cell state); only
-                       // the 1-cell shell around the tile is loaded
-};
-
-// cell l of the 1-cell shell of the 3D cell box (l < SHN): both z faces,
-// then both y faces between them, then both x faces between those
+// Source cell of the q box's entry at grid coordinates x: the cell itself;
+// 5 for coordinate -1 (left-chain halo, quirk Q8); for coordinate n the
+// right-chain stray halo (quirk Q7, halo_r_src, here in 32 bits), -1 where
+// that one is 0.  Entries further out, and those outside along two
+// directions, are in no window of an interior cell: they get some cell.
 template <int ND>
-struct Shell {
-  using L = Lay<ND>;
-  static constexpr int ZF = L::PX * L::PY, YF = L::PX * (L::PZ - 2), XF = (L::PY - 2) * (L::PZ - 2);
-  static constexpr int SHN = 2 * (ZF + YF + XF);
-  __device__ static inline void cell(int l, int& a, int& b, int& c) {
-    if (l < 2 * ZF) {
-      const int side = l >= ZF ? 1 : 0, r = l - side * ZF;
-      a = r % L::PX;
-      b = r / L::PX;
-      c = side ? L::PZ - 1 : 0;
-    } else if (l < 2 * (ZF + YF)) {
-      const int r0 = l - 2 * ZF, side = r0 >= YF ? 1 : 0, r = r0 - side * YF;
-      a = r % L::PX;
-      b = side ? L::PY - 1 : 0;
-      c = 1 + r / L::PX;
-    } else {
-      const int r0 = l - 2 * (ZF + YF), side = r0 >= XF ? 1 : 0, r = r0 - side * XF;
-      a = side ? L::PX - 1 : 0;
-      b = 1 + r % (L::PY - 2);
-      c = 1 + r / (L::PY - 2);
-    }
+__device__ __forceinline__ int q_source(const Geo& G, int x0, int x1, int x2) {
+  const int n0 = G.n[0], n1 = G.n[1], n2 = ND == 3 ? G.n[2] : 1;
+  const int y0 = x0 == -1 ? 5 : imin(imax(x0, 0), n0 - 1);
+  const int y1 = x1 == -1 ? 5 : imin(imax(x1, 0), n1 - 1);
+  const int y2 = ND == 3 ? (x2 == -1 ? 5 : imin(imax(x2, 0), n2 - 1)) : 0;
+  int c = (y2 * n1 + y1) * n0 + y0;
+  if (x0 == n0 || x1 == n1 || (ND == 3 && x2 == n2)) {
+    const int pz = ND == 3 ? x2 + 1 : 0;
+    const int h = (pz * (n1 + 2) + x1 + 1) * (n0 + 2) + x0 + 1 - (ND == 3 ? n0 * n1 : 0) - n0 - 1;
+    const int t = ((ND == 3 ? imin(pz, n2 - 1) : 0) * n1 + imin(x1 + 1, n1 - 1)) * n0 + imin(x0 + 1, n0 - 1);
+    c = h >= imax(t, 0) && h < n0 * n1 * n2 ? h : -1;
   }
-};
-
-template <int ND, typename SH>
-struct CellLoads {
-  static constexpr int NK = (Lay<ND>::PN + 255) / 256;
-  SH v[NK][ND + 1];
-};
-
-template <int ND, typename SH, bool EDGE>
-__device__ inline void cells_load(const Geo& G, const SH* __restrict__ ws, const typename OwnT<SH>::T* __restrict__ bg,
-                                  const CellBox<ND, SH>& C, const int* o, CellLoads<ND, SH>& R) {
-  using L = Lay<ND>;
-  constexpr int NK = CellLoads<ND, SH>::NK;
-  int g[NK];  // cell of each slot, -1 outside the grid (or past the box)
-#pragma unroll
-  for (int k = 0; k < NK; k++) {
-    const int l = threadIdx.x + 256 * k;
-    int a = l % L::PX, b = (l / L::PX) % L::PY, cz = l / (L::PX * L::PY);
-    if (ND == 3 && C.shell && l < Shell<ND>::SHN) Shell<ND>::cell(l, a, b, cz);
-    const int x[3] = {o[0] - 1 + a, o[1] - 1 + b, ND == 3 ? o[2] - 1 + cz : 0};
-    g[k] = l < (ND == 3 && C.shell ? Shell<ND>::SHN : L::PN) && (!EDGE || in_grid<ND>(G, x)) ? (int)cix(G, x[0], x[1], x[2]) : -1;
-  }
-#pragma unroll
-  for (int k = 0; k < NK; k++) {
-    R.v[k][0] = C.with_rho && g[k] >= 0 ? (SH)(widen(at(ws, (unsigned)g[k])) + at(bg + (long long)bRHOB() * G.N, (unsigned)g[k]))
-                                        : SH(0);
-#pragma unroll
-    for (int d = 0; d < ND; d++)
-      R.v[k][1 + d] = g[k] >= 0 ? at(ws + (long long)(C.f0 + d) * G.N, (unsigned)g[k]) : SH(0);
-  }
+  return c;
 }
 
-template <int ND, typename SH>
-__device__ inline void cells_store(const CellBox<ND, SH>& C, const CellLoads<ND, SH>& R) {
-  using L = Lay<ND>;
-#pragma unroll
-  for (int k = 0; k < CellLoads<ND, SH>::NK; k++) {
-    const int l0 = threadIdx.x + 256 * k;
-    int l = l0;
-    if (ND == 3 && C.shell) {
-      if (l0 >= Shell<ND>::SHN) continue;
-      int a, b, cz;
-      Shell<ND>::cell(l0, a, b, cz);
-      l = a + L::PX * (b + L::PY * cz);
-    }
-    if (l < L::PN) {
-      if (C.with_rho) C.CBX[l] = R.v[k][0];
-#pragma unroll
-      for (int d = 0; d < ND; d++) C.CBX[(1 + d) * L::PN + l] = R.v[k][1 + d];
-    }
-  }
-}
-
-// q box of a tile whose box crosses the grid edge (with the halo
-// substitutions): in batches of NB cells per thread, every source first,
-// then the NB loads in flight together, then the stores
-template <int ND, typename SH>
-__device__ inline void stage_q_edge(const Geo& G, const SH* __restrict__ qa, SH* __restrict__ qb, const int* o) {
-  using L = Lay<ND>;
-  constexpr int NB = ND == 3 ? 4 : 1;
+// q box of a tile whose box crosses the grid edge: in batches of NB cells
+// per thread, every source first, then the NB loads in flight together, then
+// the stores.  (A loop, to keep the code small: the edge tiles' code streams
+// through the instruction cache of every CU.)
+template <class TL, typename SH>
+__device__ __forceinline__ void stage_q_edge(const Geo& G, const SH* __restrict__ qa, SH* __restrict__ qb, const int* o) {
+  using L = Lay<TL>;
+  constexpr int ND = L::ND, NB = ND == 3 ? 4 : 1;
 #pragma unroll 1
-  for (int l0 = threadIdx.x; l0 < L::QN; l0 += 256 * NB) {
+  for (int l0 = threadIdx.x; l0 < L::QN; l0 += L::NT * NB) {
     int src[NB];
 #pragma unroll
     for (int k = 0; k < NB; k++) {
-      const int l = l0 + 256 * k;
-      src[k] = -1;
-      if (l < L::QN) {
-        const int a = l % L::QX, b = (l / L::QX) % L::QY, c = l / (L::QX * L::QY);
-        const int x[3] = {o[0] - 3 + a, o[1] - 3 + b, ND == 3 ? o[2] - 3 + c : 0};
-        src[k] = qsrc<ND>(G, x);
-      }
+      const int l = imin(l0 + L::NT * k, L::QN - 1);
+      const int a = l % L::QX, b = (l / L::QX) % L::QY, c = l / (L::QX * L::QY);
+      src[k] = q_source<ND>(G, o[0] - L::HX + a, o[1] - 3 + b, ND == 3 ? o[2] - 3 + c : 0);
     }
     SH v[NB];
 #pragma unroll
-    for (int k = 0; k < NB; k++) v[k] = src[k] >= 0 ? at(qa, (unsigned)src[k]) : (SH)0;
+    for (int k = 0; k < NB; k++) v[k] = src[k] >= 0 ? at(qa, (unsigned)src[k]) : SH(0);
 #pragma unroll
     for (int k = 0; k < NB; k++)
-      if (l0 + 256 * k < L::QN) qb[l0 + 256 * k] = v[k];
+      if (l0 + L::NT * k < L::QN) qb[l0 + L::NT * k] = v[k];
   }
 }
 
-// q box (tile + 3-cell halo) of field qa into qb, with it the cell box C
-// when C.CBX is set and a second q box (qa2 into qb2) when qa2 is set: all
-// of their loads are issued before the first store.  EDGE false: the
-// caller's tile lies at least five cells inside the grid (the box is inside)
-template <int ND, typename SH, bool EDGE>
-__device__ inline void stage_q(const Geo& G, const SH* __restrict__ qa, SH* __restrict__ qb, const int* o,
-                               const SH* __restrict__ ws = nullptr, const typename OwnT<SH>::T* __restrict__ bg = nullptr,
-                               CellBox<ND, SH> C = CellBox<ND, SH>{nullptr, false, 0}, const SH* __restrict__ qa2 = nullptr,
-                               SH* __restrict__ qb2 = nullptr) {
-  using L = Lay<ND>;
-  CellLoads<ND, SH> cl;
-  // the wave issues its staging loads at raised priority, so they leave
-  // ahead of the other workgroups' stencil arithmetic on the SIMD, and drops
-  // back once they are in flight (FP64 0.6 % faster at 256^3; the flux
-  // phase's cell loads measured slower with it)
-  __builtin_amdgcn_s_setprio(3);
-  if (C.CBX) cells_load<ND, SH, EDGE>(G, ws, bg, C, o, cl);
-  // fast path: the halo box lies inside the grid, no substitutions needed;
-  // each thread owns (a,b) columns of the box and walks their planes
-  bool inside = !EDGE || (o[0] - 3 >= 0 && o[1] - 3 >= 0 && o[0] + L::TX + 3 <= G.n[0] && o[1] + L::TY + 3 <= G.n[1]);
-  if (EDGE && ND == 3) inside = inside && o[2] - 3 >= 0 && o[2] + L::TZ + 3 <= G.n[2];
-  if (inside) {
-    constexpr int PL = L::QX * L::QY, NKF = (PL + 255) / 256;
+// q box (tile + 3-cell halo) of one field on its way to LDS: load() issues
+// this thread's global loads, store() writes them (of an edge tile store()
+// does both).  Each thread owns columns
+// along dim 2 of XC neighbouring cells, and, where the workgroup has threads
+// enough, a part of the planes.
+template <class TL, typename SH, bool EDGE>
+struct QBox {
+  using L = Lay<TL>;
+  static constexpr int ND = L::ND, XC = L::XC;
+  static constexpr int NPC = L::QX / XC * L::QY;                 // columns
+  static constexpr int NKF = (NPC + L::NT - 1) / L::NT;          // columns per thread
+  static constexpr int NG = imax(1, L::NT / NPC);                // parts of the planes
+  static constexpr int PG = L::QZ / NG;                          // planes per part
+  static_assert(PG * NG == L::QZ, "the parts are equal");
+  SH v[NKF][PG][XC];
+
+  __device__ static __forceinline__ bool inside(const Geo& G, const int* o) {
+    if (!EDGE) return true;
+    bool in = o[0] >= L::HX && o[1] >= 3 && o[0] + L::TX + L::HX <= G.n[0] && o[1] + L::TY + 3 <= G.n[1];
+    if (ND == 3) in = in && o[2] >= 3 && o[2] + L::TZ + 3 <= G.n[2];
+    return in;
+  }
+  // (threads without a column load one again, so the loads are
+  // unconditional and their registers have no other definition to merge)
+  __device__ __forceinline__ void get(const Geo& G, const SH* __restrict__ qa, const int* o) {
     const unsigned zs = (unsigned)G.n[0] * (unsigned)G.n[1];
-    SH v[NKF][L::QZ], v2[NKF][L::QZ];
 #pragma unroll
     for (int k = 0; k < NKF; k++) {
-      const int l = threadIdx.x + 256 * k;
-      if (l < PL) {
-        const int a = l % L::QX, b = l / L::QX;
-        const unsigned g0 = cix(G, o[0] - 3 + a, o[1] - 3 + b, ND == 3 ? o[2] - 3 : 0);
+      const int t = threadIdx.x + L::NT * k;
+      const int gt = NG > 1 ? t / NPC : 0, g = gt < NG ? gt : 0, lt = t - gt * NPC, l = lt < NPC ? lt : 0;
+      const int a = XC * (l % (L::QX / XC)), b = l / (L::QX / XC);
+      // the box's far edges and corners are in no window: their columns load
+      // values that others load anyway
+      const bool yin = b >= 2 && b < L::TY + 4;
+      const int xa = yin ? a : imin(imax(a, L::HX - XC), L::HX + L::TX);
+      const bool out = ND == 3 && !(yin && a >= L::HX - XC && a <= L::HX + L::TX);
+      const bool lo = out && g == 0, hi = out && g == NG - 1;
+      const unsigned g0 = cix(G, o[0] - L::HX + xa, o[1] - 3 + b, ND == 3 ? o[2] - 3 + g * PG : 0);
 #pragma unroll
-        for (int cz = 0; cz < L::QZ; cz++) v[k][cz] = at(qa, g0 + cz * zs);
-        if (qa2) {
+      for (int c = 0; c < PG; c++) {
+        unsigned z = c * zs;
+        if (ND == 3 && c < 2) z = lo ? 2 * zs : z;
+        if (ND == 3 && c >= PG - 2) z = hi ? (PG - 3) * zs : z;
+        ldg<XC>(qa, g0 + z, v[k][c]);
+      }
+    }
+  }
+  __device__ __forceinline__ void put(SH* __restrict__ qb) {
 #pragma unroll
-          for (int cz = 0; cz < L::QZ; cz++) v2[k][cz] = at(qa2, g0 + cz * zs);
+    for (int k = 0; k < NKF; k++) {
+      const int t = threadIdx.x + L::NT * k;
+      const int g = NG > 1 ? t / NPC : 0, l = t - g * NPC;
+      if (g < NG && l < NPC) {
+        const int a = XC * (l % (L::QX / XC)), b = l / (L::QX / XC);
+#pragma unroll
+        for (int c = 0; c < PG; c++) stl<XC>(qb + a + L::QX * (b + L::QY * (g * PG + c)), v[k][c]);
+      }
+    }
+  }
+  __device__ __forceinline__ void load(const Geo& G, const SH* __restrict__ qa, const int* o) {
+    if constexpr (!EDGE) get(G, qa, o);
+  }
+  __device__ __forceinline__ void store(const Geo& G, const SH* __restrict__ qa, SH* __restrict__ qb, const int* o) {
+    if constexpr (!EDGE) {
+      put(qb);
+    } else if (inside(G, o)) {
+      get(G, qa, o);
+      put(qb);
+    } else {
+      stage_q_edge<TL, SH>(G, qa, qb, o);
+    }
+  }
+};
+
+// rho_t = rho + rho_b on the tile + 1-cell halo (the sum in the background's
+// precision, rounded to the stencils'); cells outside the grid hold 0
+template <class TL, typename SH, bool EDGE>
+__device__ __forceinline__ void stage_rho_t(const Geo& G, const SH* __restrict__ ws, const typename OwnT<SH>::T* __restrict__ bg,
+                                   SH* __restrict__ cb, const int* o) {
+  using L = Lay<TL>;
+  using OT = typename OwnT<SH>::T;
+  constexpr int ND = L::ND, XC = L::XC, NC = L::PN / XC, NK = (NC + L::NT - 1) / L::NT;
+  const OT* __restrict__ rb = bg + (long long)bRHOB() * G.N;
+  SH r[NK][XC];
+  OT b[NK][XC];
+#pragma unroll
+  for (int k = 0; k < NK; k++) {
+    const int l = threadIdx.x + L::NT * k;
+    const int a = XC * (l % (L::PX / XC)), q = l / (L::PX / XC);
+    const int x[3] = {o[0] - L::RX + a, o[1] - 1 + q % L::PY, ND == 3 ? o[2] - 1 + q / L::PY : 0};
+    if (l < NC) {
+      if (!EDGE) {
+        const unsigned c = cix(G, x[0], x[1], x[2]);
+        ldg<XC>(ws, c, r[k]);
+        ldg<XC>(rb, c, b[k]);
+      } else {
+#pragma unroll
+        for (int u = 0; u < XC; u++) {
+          const int y[3] = {x[0] + u, x[1], x[2]};
+          const bool in = in_grid<ND>(G, y);
+          const unsigned c = in ? cix(G, y[0], y[1], y[2]) : 0u;
+          r[k][u] = in ? at(ws, c) : SH(0);
+          b[k][u] = in ? at(rb, c) : OT(0.0);
         }
       }
     }
-    __builtin_amdgcn_s_setprio(0);
-    if (C.CBX) cells_store<ND, SH>(C, cl);
+  }
 #pragma unroll
-    for (int k = 0; k < NKF; k++) {
-      const int l = threadIdx.x + 256 * k;
-      if (l < PL) {
+  for (int k = 0; k < NK; k++) {
+    const int l = threadIdx.x + L::NT * k;
+    if (l < NC) {
+      SH s[XC];
 #pragma unroll
-        for (int cz = 0; cz < L::QZ; cz++) qb[cz * PL + l] = v[k][cz];
-        if (qa2) {
-#pragma unroll
-          for (int cz = 0; cz < L::QZ; cz++) qb2[cz * PL + l] = v2[k][cz];
-        }
-      }
+      for (int u = 0; u < XC; u++) s[u] = (SH)(widen(r[k][u]) + b[k][u]);
+      stl<XC>(cb + XC * l, s);
     }
-    return;
   }
-  if constexpr (EDGE) {
-    if (C.CBX) cells_store<ND, SH>(C, cl);
-    stage_q_edge<ND, SH>(G, qa, qb, o);
-    if (qa2) stage_q_edge<ND, SH>(G, qa2, qb2, o);
-  }
-  __builtin_amdgcn_s_setprio(0);
 }
 
-// The terms of one tile whose origin (first interior cell) is o.  EDGE
-// false: every cell of the tile lies in [5, n-6] along every direction, so
-// no cell of it or of its halos is a ghost or on a zeroed layer, every
-// staged box lies inside the grid and no cell has a ghost image; the
-// boundary checks are then compiled out (the arithmetic is the same).  The
-// own cell's interior test stays a run-time test in both bodies: known true,
-// it lets the compiler keep values loaded in one phase live through later
-// ones, and the FP64 kernel then spills (336 bytes per lane at gfx950).
-template <int ND, typename SH, bool EDGE>
-__device__ __forceinline__ void rhs_tile(const Geo& G, const RhsArgs& A, SH* __restrict__ sm, const int* o) {
-  using L = Lay<ND>;
-  using AT = SH;  // arithmetic type of the stencils
-  // own-cell type: FP64 (the own-cell update and the RK combination are
-  // FP64 with FP32 stencils too), Dual in the tangent-linear step
-  using OT = typename OwnT<SH>::T;
-  constexpr int NP = L::NP;
-  constexpr int TX = L::TX, TY = L::TY, TZ = L::TZ;
-  const int tid = threadIdx.x;
-  const int lc[3] = {tid % TX, (tid / TX) % TY, ND == 3 ? tid / (TX * TY) : 0};
-  int x[3] = {o[0] + lc[0], o[1] + lc[1], o[2] + lc[2]};
-  const bool valid = interior_c<ND>(G, x);
-  const long long N = G.N;
-  const unsigned c = cix(G, x[0], x[1], x[2]);  // own cell (used by valid threads only)
-  const OT* __restrict__ w = (const OT*)A.win;    // own-cell values
-  const SH* __restrict__ ws = (const SH*)A.wsh;    // neighbour values (stencil precision)
-  const OT* __restrict__ bg = (const OT*)A.bg;  // background (Dual in the tangent-linear step)
-  const SH* __restrict__ pr = (const SH*)A.prim;
-  const unsigned T = G.terms;
-  AT acc[NP];
+// The window of a thread's cells along direction D (0, 1, 2) of a q box:
+// the values at offsets -2..2 of each cell and nu_{i+1/2}, nu_{i-1/2} (sc =
+// delx * cmax * chyp).  The coefficient of an interface is a ratio of its own
+// (see nu_ratio), so two neighbours along dim 0 share the one between them.
+template <class TL, typename SH>
+struct Win {
+  using V = typename ValT<SH>::T;
+  static constexpr int XC = TL::XC;
+  SH q[XC][5];
+  V nr[XC], nl[XC];
+  template <int D>
+  __device__ __forceinline__ void load(const SH* __restrict__ qb, int qc, int s, const V* sc) {
+    if constexpr (D == 0 && XC == 2) {
+      SH w[10];
 #pragma unroll
-  for (int f = 0; f < NP; f++) acc[f] = AT(0);
-  AT dx[ND], rdx[ND];
+      for (int k = 0; k < 10; k += 2) ldl<2>(qb + qc - 4 + k, w + k);
+      V y[8];
 #pragma unroll
-  for (int d = 0; d < ND; d++) {
-    if (A.dx1) {  // tensor-product grid: one spacing per coordinate
-      const int od = d == 0 ? 0 : (d == 1 ? G.n[0] : G.n[0] + G.n[1]);
-      dx[d] = valid ? (AT)A.dx1[od + x[d]] : AT(1);
-      rdx[d] = valid ? (AT)A.rdx1[od + x[d]] : AT(1);
+      for (int k = 0; k < 8; k++) y[k] = valof(w[k + 1]);
+      V R[3];
+      nu_ratios<3>(y, R);
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+#pragma unroll
+        for (int k = 0; k < 5; k++) q[u][k] = w[2 + u + k];
+        nl[u] = sc[u] * R[u];
+        nr[u] = sc[u] * R[u + 1];
+      }
     } else {
-      dx[d] = valid ? (AT)at(A.delx + (long long)d * N, c) : AT(1);
-      rdx[d] = valid ? (AT)at(A.rdelx + (long long)d * N, c) : AT(1);
+      SH w[7][XC];
+#pragma unroll
+      for (int k = 0; k < 7; k++) ldl<XC>(qb + qc + (k - 3) * s, w[k]);
+#pragma unroll
+      for (int u = 0; u < XC; u++) {
+        V y[7];
+#pragma unroll
+        for (int k = 0; k < 7; k++) y[k] = valof(w[k][u]);
+        V R[2];
+        nu_ratios<2>(y, R);
+        nl[u] = sc[u] * R[0];
+        nr[u] = sc[u] * R[1];
+#pragma unroll
+        for (int k = 0; k < 5; k++) q[u][k] = w[1 + k][u];
+      }
     }
   }
+};
 
-  AT* const SDX = sm + L::CB + L::SHR;  // spacing table (tensor-product grids)
-  if (A.dx1 && tid < L::DXT) {  // visible after the first barrier
-    const int d = tid < TX ? 0 : (tid < TX + TY ? 1 : 2);
-    const int xx = o[d] + tid - (d == 0 ? 0 : (d == 1 ? TX : TX + TY));
-    const int od = d == 0 ? 0 : (d == 1 ? G.n[0] : G.n[0] + G.n[1]);
-    const bool ing = d < ND && xx < G.n[d];
-    SDX[tid] = ing ? (AT)A.dx1[od + xx] : AT(1);
-    SDX[L::DXT + tid] = ing ? (AT)A.rdx1[od + xx] : AT(1);
-  }
-
-  AT* const CBX = sm;  // cell box (tile + 1)
-  const int pc = (lc[0] + 1) + L::PX * ((lc[1] + 1) + L::PY * (ND == 3 ? lc[2] + 1 : 0));
-  const int ps[3] = {1, L::PX, L::PX * L::PY};
-  const bool want_mom = G.hyper && (T & SMAUG_T_HMOM);
-  const bool want_eterm = (T & SMAUG_T_ETERM) != 0;
-
-  // FP64 3D: the flux phase's own-cell state fills the tile's cells of the
-  // momentum phases' cell box (the same rho + rho_b sum as the staging), so
-  // that staging loads only the box's shell
-  const bool own_cb = sizeof(SH) == 8 && ND == 3 && want_mom && (T & SMAUG_T_FLUX);
-  // ------------------------------------------------------------ fluxes
-  if (T & SMAUG_T_FLUX) {
-    AT* FB = sm + L::CB;
-    // the thread's own tile cell: its state is loaded once for every
-    // direction (and the flux function's v, p_t, ... of it are shared); a
-    // second slot per direction covers the 2 + 2 halo layers along it
-    const bool in0 = !EDGE || in_grid<ND>(G, x);
-    CellState<ND, AT> S0;
-    if (in0) load_cell<ND, SH, AT>(G, ws, bg, c, S0);
-    if (own_cb) {  // the tile's cells of the momentum phases' cell box: rho_t, m
-      CBX[pc] = in0 ? S0.rho + S0.rhob : AT(0);
-#pragma unroll
-      for (int q = 0; q < ND; q++) CBX[(1 + q) * L::PN + pc] = in0 ? S0.m[q] : AT(0);
-    }
-#pragma unroll
-    for (int d = 0; d < ND; d++) {
-      const int ex[3] = {d == 0 ? 2 : 0, d == 1 ? 2 : 0, d == 2 ? 2 : 0};
-      const int rx = TX + 2 * ex[0], ry = TY + 2 * ex[1];
-      const int Td = d == 0 ? TX : (d == 1 ? TY : TZ);
-      const int pa = d == 0 ? 1 : 0, qa = d == 2 ? 1 : 2;  // the other two axes
-      const int Tp = pa == 0 ? TX : TY;
-      const int Fd = Tp * (ND == 3 ? (qa == 1 ? TY : TZ) : 1);  // face of the tile across d
-      static_assert(ND == 3 ? 4 * TY * TZ <= 256 && 4 * TX * TZ <= 256 && 4 * TX * TY <= 256
-                            : 4 * TX <= 256 && 4 * TY <= 256,
-                    "the halo layers of a direction fit one slot per thread");
-      CellState<ND, AT> S1;
-      bool in1 = false;
-      int l1 = 0;
-      const bool h1 = tid < 4 * Fd;
-      if (h1) {
-        const int layer = tid / Fd, r = tid - layer * Fd;
-        int rc[3] = {0, 0, 0};
-        rc[d] = layer < 2 ? layer : Td + layer;  // region coordinates 0, 1 and Td+2, Td+3
-        rc[pa] = r % Tp;
-        if (ND == 3) rc[qa] = r / Tp;
-        const int xr[3] = {o[0] - ex[0] + rc[0], o[1] - ex[1] + rc[1], ND == 3 ? o[2] - ex[2] + rc[2] : 0};
-        in1 = !EDGE || in_grid<ND>(G, xr);
-        l1 = rc[0] + rx * (rc[1] + ry * rc[2]);
-        if (in1) load_cell<ND, SH, AT>(G, ws, bg, cix(G, xr[0], xr[1], xr[2]), S1);
-      }
-      {
-        AT F[NP];
-        if (in0) {
-          fluxes_of<ND, AT>(G, S0, d, F);
-        } else {
-#pragma unroll
-          for (int f = 0; f < NP; f++) F[f] = AT(0);
-        }
-        const int l0 = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
-        // the flux of b_d along d is zero: its slot is neither written nor read
-#pragma unroll
-        for (int f = 0; f < NP; f++)
-          if (f != fB(ND, d)) FB[f * L::FN + l0] = F[f];
-      }
-      if (h1) {
-        AT F[NP];
-        if (in1) {
-          fluxes_of<ND, AT>(G, S1, d, F);
-        } else {
-#pragma unroll
-          for (int f = 0; f < NP; f++) F[f] = AT(0);
-        }
-#pragma unroll
-        for (int f = 0; f < NP; f++)
-          if (f != fB(ND, d)) FB[f * L::FN + l1] = F[f];
-      }
-      __syncthreads();
-      if (valid && !z4e<EDGE>(G, zFLUX(ND), d, x[d])) {
-        const int s = d == 0 ? 1 : (d == 1 ? rx : rx * ry);
-        const int li = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
-        const AT inv = rdx[d] * AT(1.0 / 12.0);
-#pragma unroll
-        for (int f = 0; f < NP; f++) {
-          if (f == fB(ND, d)) continue;
-          const AT* Fp = FB + f * L::FN + li;
-          acc[f] -= ((8 * Fp[s] - 8 * Fp[-s]) + (Fp[-2 * s] - Fp[2 * s])) * inv;
-        }
-      }
-      __syncthreads();
-    }
-  }
-
-  const OT rho_c = valid ? at(w, c) : OT(0.0);
-  const OT rhob_c = valid ? at(bg + (long long)bRHOB() * N, c) : OT(1.0);
-  const AT rt_c = (AT)(rho_c + rhob_c);
-
-  // ------------------------------------------------------------ hyperdiffusion + energy terms
-  SH* qb = sm + L::CB;                                 // q box
-  AT* NR = sm + L::CB + L::QN;                         // region arrays
-  AT* RG[4] = {NR, NR + L::RN, NR + 2 * L::RN, NR + 3 * L::RN};  // GA/GB of the two cross directions
-  // tile-cell index in the q box and its strides
-  const int qc = (lc[0] + 3) + L::QX * ((lc[1] + 3) + L::QY * (ND == 3 ? lc[2] + 3 : 0));
-  const int qs[3] = {1, L::QX, L::QX * L::QY};
-
-  AT cm[ND];
-#pragma unroll
-  for (int d = 0; d < ND; d++) cm[d] = (AT)__longlong_as_double((long long)A.cmax_bits[d]);
-
-  // rho (src/hyperdifrhosource1.cu) and e_int (src/hyperdifesource1.cu):
-  // both boxes are staged in one round trip, the e_int box after the rho box
-  const bool h_rho = G.hyper && (T & SMAUG_T_HRHO), h_e = G.hyper && (T & SMAUG_T_HE);
-  static_assert(2 * L::QN <= L::SHR, "two q boxes in the shared area");
-  if (h_rho || h_e) {
-    const SH* qe = pr + (long long)pQE(ND) * N;
-    SH* qbe = h_rho ? qb + L::QN : qb;
-    stage_q<ND, SH, EDGE>(G, h_rho ? ws : qe, qb, o, ws, bg, CellBox<ND, SH>{nullptr, false, 0}, h_rho && h_e ? qe : nullptr,
-                    h_rho && h_e ? qbe : nullptr);
-    __syncthreads();
-    if (valid && h_rho) {
-#pragma unroll
-      for (int dim = 0; dim < ND; dim++) {
-        AT nur, nul;
-        nu_win<SH, AT>(qb, qc, qs[dim], dx[dim] * cm[dim] * (AT)G.chyp[fRHO()], nur, nul);
-        const bool z = z1e<EDGE>(G, zRHO, dim, x[dim]);
-        const AT q0 = qb[qc];
-        const AT gr = z ? AT(0) : (qb[qc + qs[dim]] - q0) * rdx[dim];
-        const AT gl = z ? AT(0) : (q0 - qb[qc - qs[dim]]) * rdx[dim];
-        acc[fRHO()] += (nur * gr - nul * gl) * rdx[dim];
-      }
-    }
-    if (valid && h_e) {
-#pragma unroll
-      for (int dim = 0; dim < ND; dim++) {
-        AT nur, nul;
-        nu_win<SH, AT>(qbe, qc, qs[dim], dx[dim] * cm[dim] * (AT)G.chyp[fE(ND)], nur, nul);
-        const bool z = z1e<EDGE>(G, zTMP1, dim, x[dim]);
-        const AT q0 = qbe[qc];
-        const AT gr = z ? AT(0) : (qbe[qc + qs[dim]] - q0) * rdx[dim];
-        const AT gl = z ? AT(0) : (q0 - qbe[qc - qs[dim]]) * rdx[dim];
-        acc[fE(ND)] += (nur * gr - nul * gl) * rdx[dim];
-      }
-    }
-    __syncthreads();
-  }
-
-  AT ptb = AT(0), bbc[ND];  // background terms, formed in FP64
-  if (want_eterm && valid) {
-    OT bb2 = OT(0.0), bbd[ND];
-#pragma unroll
-    for (int d = 0; d < ND; d++) {
-      bbd[d] = at(bg + (long long)bBB(d) * N, c);
-      bbc[d] = (AT)bbd[d];
-      bb2 = d == 0 ? bbd[d] * bbd[d] : bb2 + bbd[d] * bbd[d];
-    }
-    ptb = (AT)((G.gamma - 1) * at(bg + (long long)bEB() * N, c) - 0.5 * (G.gamma - 2) * bb2);
-  }
-
-  // momentum phases (q = v_f): energy terms, diagonal and off-diagonal sources
-  if (want_mom || want_eterm) {
-#pragma unroll
-    for (int f = 0; f < ND; f++) {
-      // the first box brings rho_t and m on the cell box with it
-      stage_q<ND, SH, EDGE>(G, pr + (long long)pV(f) * N, qb, o, ws, bg,
-                      CellBox<ND, SH>{f == 0 && want_mom ? CBX : nullptr, true, fMOM(0), own_cb});
-      __syncthreads();
-      if (want_eterm && valid) {  // addenergyterms_cd2 for dir f
-        AT gf[ND];
-#pragma unroll
-        for (int i2 = 0; i2 < ND; i2++) {
-          const int s = qs[i2];
-          gf[i2] = z4e<EDGE>(G, zVEL(f), i2, x[i2])
-                       ? AT(0)
-                       : ((8 * qb[qc + s] - 8 * qb[qc - s]) + (qb[qc - 2 * s] - qb[qc + 2 * s])) * (rdx[i2] * AT(1.0 / 12.0));
-        }
-        AT t = -ptb * gf[f];
-#pragma unroll
-        for (int i2 = 0; i2 < ND; i2++) t += bbc[i2] * bbc[f] * gf[i2];
-        acc[fE(ND)] += t;
-      }
-      if (want_mom) {
-        // one region pass per f for both cross directions: the tile
-        // extended by one layer along f, products rho_t*t6 and t6*m_d for
-        // each d != f; the own cell's nu in every direction stays in
-        // registers (src/hyperdifmomsource1.cu, src/hyperdifmomsourcene1.cu)
-        const int ex[3] = {f == 0 ? 1 : 0, f == 1 ? 1 : 0, f == 2 ? 1 : 0};
-        const int rx = TX + 2 * ex[0], ry = TY + 2 * ex[1];
-        const int sf = f == 0 ? 1 : (f == 1 ? rx : rx * ry);
-        const int ri = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
-        const AT Kc = (AT)G.chyp[fMOM(f)];
-        AT nur[ND], nul[ND];
-#pragma unroll
-        for (int d = 0; d < ND; d++) {
-          nur[d] = nul[d] = AT(0);
-          if (valid) nu_win<SH, AT>(qb, qc, qs[d], dx[d] * cm[d] * Kc, nur[d], nul[d]);
-          if (d != f) {
-            const int k = d < f ? d : d - 1;
-            AT g7 = 0, g8 = 0;
-            if (valid) {
-              const AT t5 =
-                  z1e<EDGE>(G, zTMP4, d, x[d]) ? AT(0) : (qb[qc + qs[d]] - qb[qc - qs[d]]) * rdx[d] * AT(0.5);
-              const AT t6 = t5 * (nur[d] + nul[d]) * AT(0.25);
-              g7 = rt_c * t6;
-              g8 = t6 * CBX[(1 + d) * L::PN + pc];
-            }
-            RG[2 * k][ri] = g7;
-            RG[2 * k + 1][ri] = g8;
-          }
-        }
-        {  // the two layers just outside the tile along f
-          const int pd = f == 0 ? 1 : 0, qd = f == 2 ? 1 : 2;
-          const int Tp = pd == 0 ? TX : TY, Tq = ND == 3 ? (qd == 1 ? TY : TZ) : 1;
-          const int Fc = Tp * Tq;
-          // FP64: one (border cell, cross direction) task per thread, 2 Fc
-          // (ND-1) <= 256 tasks; kt is uniform per wavefront (2 Fc is 64 or
-          // 128 in 3D), so each wavefront runs one direction's body (measured
-          // 2 % faster at 256^3).  FP32: one border cell per thread for all
-          // cross directions (the split measured 1.6 % slower there).
-          constexpr int NTK = sizeof(AT) == 8 ? ND - 1 : 1;
-          if (tid < 2 * Fc * NTK) {
-            const int kt = NTK > 1 ? tid / (2 * Fc) : -1, r2 = tid - (NTK > 1 ? kt * 2 * Fc : 0);
-            const int side = r2 >= Fc ? 1 : 0, r = r2 - side * Fc;
-            int bc[3] = {0, 0, 0};
-            bc[f] = side ? (f == 0 ? TX : (f == 1 ? TY : TZ)) + 1 : 0;
-            bc[pd] = r % Tp;
-            if (ND == 3) bc[qd] = r / Tp;
-            const int l = bc[0] + rx * (bc[1] + ry * bc[2]);
-            const int rel[3] = {bc[0] - ex[0], bc[1] - ex[1], ND == 3 ? bc[2] - ex[2] : 0};
-            int xr[3] = {o[0] + rel[0], o[1] + rel[1], ND == 3 ? o[2] + rel[2] : 0};
-            const bool in = !EDGE || interior_c<ND>(G, xr);
-            const unsigned gq = in ? cix(G, xr[0], xr[1], xr[2]) : 0u;
-            const int pi = (rel[0] + 1) + L::PX * ((rel[1] + 1) + L::PY * (ND == 3 ? rel[2] + 1 : 0));
-            const AT rt = in ? CBX[pi] : AT(0);
-            const int qi = (rel[0] + 3) + L::QX * ((rel[1] + 3) + L::QY * (ND == 3 ? rel[2] + 3 : 0));
-#pragma unroll
-            for (int d = 0; d < ND; d++) {
-              if (d == f) continue;
-              const int k = d < f ? d : d - 1;
-              if (NTK > 1 && k != kt) continue;
-              AT g7 = 0, g8 = 0;
-              if (in) {
-                // d != f: the border cell's coordinate along d is a tile coordinate
-                const int ti = (d == 0 ? 0 : (d == 1 ? TX : TX + TY)) + rel[d];
-                const AT dxr = A.dx1 ? SDX[ti] : (AT)at(A.delx + (long long)d * N, gq);
-                const AT rdxr = A.dx1 ? SDX[L::DXT + ti] : (AT)at(A.rdelx + (long long)d * N, gq);
-                AT nr, nl;
-                nu_win<SH, AT>(qb, qi, qs[d], dxr * cm[d] * Kc, nr, nl);
-                const AT t5 =
-                    z1e<EDGE>(G, zTMP4, d, xr[d]) ? AT(0) : (qb[qi + qs[d]] - qb[qi - qs[d]]) * rdxr * AT(0.5);
-                const AT t6 = t5 * (nr + nl) * AT(0.25);
-                g7 = rt * t6;
-                g8 = t6 * CBX[(1 + d) * L::PN + pi];
-              }
-              RG[2 * k][l] = g7;
-              RG[2 * k + 1][l] = g8;
-            }
-          }
-        }
-        __syncthreads();
-        if (valid) {
-          const AT* mf = CBX + (1 + f) * L::PN + pc;
-          const AT mc = mf[0];
-#pragma unroll
-          for (int d = 0; d < ND; d++) {
-            const int s = qs[d];
-            const int sp = ps[d];
-            const bool z = z1e<EDGE>(G, zTMP4, d, x[d]);
-            const AT q0 = qb[qc];
-            const AT gr = z ? AT(0) : (qb[qc + s] - q0) * rdx[d];
-            const AT gl = z ? AT(0) : (q0 - qb[qc - s]) * rdx[d];
-            const AT rtp = CBX[pc + sp], rtm = CBX[pc - sp];
-            const AT rr = (rt_c + rtp) * AT(0.5), rl = (rt_c + rtm) * AT(0.5);
-            const AT mr = (mc + mf[sp]) * AT(0.5), ml = (mc + mf[-sp]) * AT(0.5);
-            const AT dmv = (rr * nur[d] * gr - rl * nul[d] * gl) * (rdx[d] * AT(0.5));
-            const AT dev = (mr * nur[d] * gr - ml * nul[d] * gl) * (rdx[d] * AT(0.5));
-            acc[fMOM(f)] += dmv;
-            acc[fE(ND)] += dev;
-            if (d == f) {
-              acc[fMOM(f)] += dmv;
-              acc[fE(ND)] += dev;
-            } else {
-              const int k = d < f ? d : d - 1;
-              const AT* GAk = RG[2 * k];
-              const AT* GBk = RG[2 * k + 1];
-              const AT o7 = z1e<EDGE>(G, zTMP7, f, x[f]) ? AT(0) : (GAk[ri + sf] - GAk[ri - sf]) * (rdx[f] * AT(0.5));
-              const AT o8 = z1e<EDGE>(G, zTMP8, f, x[f]) ? AT(0) : (GBk[ri + sf] - GBk[ri - sf]) * (rdx[f] * AT(0.5));
-              acc[fMOM(d)] += o7;
-              acc[fE(ND)] += o8;
-            }
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
-
-  // magnetic phases (q = b_f): curl-form cross terms (sb = -1,
-  // src/hyperdifbsourcene1.cu) and diagonal terms (sb = +1,
-  // src/hyperdifbsource1.cu), one region pass per f for both d != f
-  if (G.hyper && (T & SMAUG_T_HB)) {
-#pragma unroll
-    for (int f = 0; f < ND; f++) {
-      // the first box brings b on the cell box with it (the momentum
-      // phases are done with the cell box: each ended with a barrier)
-      stage_q<ND, SH, EDGE>(G, ws + (long long)fB(ND, f) * N, qb, o, ws, bg,
-                      CellBox<ND, SH>{f == 0 ? CBX : nullptr, false, fB(ND, 0)});
-      __syncthreads();
-      const int ex[3] = {f == 0 ? 1 : 0, f == 1 ? 1 : 0, f == 2 ? 1 : 0};
-      const int rx = TX + 2 * ex[0], ry = TY + 2 * ex[1];
-      const int sf = f == 0 ? 1 : (f == 1 ? rx : rx * ry);
-      const int ri = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
-      const AT Kc = (AT)G.chyp[fB(ND, f)];
-      AT nur[ND], nul[ND];
-#pragma unroll
-      for (int d = 0; d < ND; d++) {
-        nur[d] = nul[d] = AT(0);
-        if (d == f) continue;
-        const int k = d < f ? d : d - 1;
-        AT g3 = 0, g5 = 0;
-        if (valid) {
-          nu_win<SH, AT>(qb, qc, qs[d], dx[d] * cm[d] * Kc, nur[d], nul[d]);
-          const AT t2 =
-              z1e<EDGE>(G, zTMP1, d, x[d]) ? AT(0) : (qb[qc + qs[d]] - qb[qc - qs[d]]) * rdx[d] * AT(0.5);
-          const AT t3 = t2 * (nul[d] + nur[d]) * AT(0.5);
-          g3 = t3;
-          g5 = t3 * CBX[(1 + d) * L::PN + pc];
-        }
-        RG[2 * k][ri] = g3;
-        RG[2 * k + 1][ri] = g5;
-      }
-      {  // the two layers just outside the tile along f
-        const int pd = f == 0 ? 1 : 0, qd = f == 2 ? 1 : 2;
-        const int Tp = pd == 0 ? TX : TY, Tq = ND == 3 ? (qd == 1 ? TY : TZ) : 1;
-        const int Fc = Tp * Tq;
-        // FP64: one (border cell, cross direction) task per thread, 2 Fc
-        // (ND-1) <= 256 tasks; kt is uniform per wavefront (2 Fc is 64 or
-        // 128 in 3D), so each wavefront runs one direction's body (measured
-        // 2 % faster at 256^3).  FP32: one border cell per thread for all
-        // cross directions (the split measured 1.6 % slower there).
-        constexpr int NTK = sizeof(AT) == 8 ? ND - 1 : 1;
-        if (tid < 2 * Fc * NTK) {
-          const int kt = NTK > 1 ? tid / (2 * Fc) : -1, r2 = tid - (NTK > 1 ? kt * 2 * Fc : 0);
-          const int side = r2 >= Fc ? 1 : 0, r = r2 - side * Fc;
-          int bc[3] = {0, 0, 0};
-          bc[f] = side ? (f == 0 ? TX : (f == 1 ? TY : TZ)) + 1 : 0;
-          bc[pd] = r % Tp;
-          if (ND == 3) bc[qd] = r / Tp;
-          const int l = bc[0] + rx * (bc[1] + ry * bc[2]);
-          const int rel[3] = {bc[0] - ex[0], bc[1] - ex[1], ND == 3 ? bc[2] - ex[2] : 0};
-          int xr[3] = {o[0] + rel[0], o[1] + rel[1], ND == 3 ? o[2] + rel[2] : 0};
-          const bool in = !EDGE || interior_c<ND>(G, xr);
-          const unsigned gq = in ? cix(G, xr[0], xr[1], xr[2]) : 0u;
-          const int pi = (rel[0] + 1) + L::PX * ((rel[1] + 1) + L::PY * (ND == 3 ? rel[2] + 1 : 0));
-          const int qi = (rel[0] + 3) + L::QX * ((rel[1] + 3) + L::QY * (ND == 3 ? rel[2] + 3 : 0));
-#pragma unroll
-          for (int d = 0; d < ND; d++) {
-            if (d == f) continue;
-            const int k = d < f ? d : d - 1;
-            if (NTK > 1 && k != kt) continue;
-            AT g3 = 0, g5 = 0;
-            if (in) {
-              // d != f: the border cell's coordinate along d is a tile coordinate
-              const int ti = (d == 0 ? 0 : (d == 1 ? TX : TX + TY)) + rel[d];
-              const AT dxr = A.dx1 ? SDX[ti] : (AT)at(A.delx + (long long)d * N, gq);
-              const AT rdxr = A.dx1 ? SDX[L::DXT + ti] : (AT)at(A.rdelx + (long long)d * N, gq);
-              AT nr, nl;
-              nu_win<SH, AT>(qb, qi, qs[d], dxr * cm[d] * Kc, nr, nl);
-              const AT t2 =
-                  z1e<EDGE>(G, zTMP1, d, xr[d]) ? AT(0) : (qb[qi + qs[d]] - qb[qi - qs[d]]) * rdxr * AT(0.5);
-              const AT t3 = t2 * (nl + nr) * AT(0.5);
-              g3 = t3;
-              g5 = t3 * CBX[(1 + d) * L::PN + pi];
-            }
-            RG[2 * k][l] = g3;
-            RG[2 * k + 1][l] = g5;
-          }
-        }
-      }
-      __syncthreads();
-      if (valid) {
-#pragma unroll
-        for (int d = 0; d < ND; d++) {
-          if (d == f) continue;
-          const int k = d < f ? d : d - 1;
-          const AT* GAk = RG[2 * k];
-          const AT* GBk = RG[2 * k + 1];
-          const AT o3 = z1e<EDGE>(G, zTMP3, f, x[f]) ? AT(0) : (GAk[ri + sf] - GAk[ri - sf]) * (rdx[f] * AT(0.5));
-          const AT o5 = z1e<EDGE>(G, zTMP5, f, x[f]) ? AT(0) : (GBk[ri + sf] - GBk[ri - sf]) * (rdx[f] * AT(0.5));
-          acc[fB(ND, d)] += -o3;
-          acc[fE(ND)] += -o5;
-          const int s = qs[d];
-          const bool z = z1e<EDGE>(G, zTMP1, d, x[d]);
-          const AT q0 = qb[qc];
-          const AT gr = z ? AT(0) : (qb[qc + s] - q0) * rdx[d];
-          const AT gl = z ? AT(0) : (q0 - qb[qc - s]) * rdx[d];
-          const AT br = (q0 + qb[qc + s]) * AT(0.5), bl = (q0 + qb[qc - s]) * AT(0.5);
-          acc[fB(ND, f)] += (gr * nur[d] - gl * nul[d]) * rdx[d];
-          acc[fE(ND)] += (br * gr * nur[d] - bl * gl * nul[d]) * rdx[d];
-        }
-      }
-      __syncthreads();
-    }
-  }
-
-  if (!valid) return;
-  // ------------------------------------------------------------ gravity
-  if (T & SMAUG_T_GRAV) {
-#pragma unroll
-    for (int d = 0; d < ND; d++) {
-      if (G.g[d] == 0.0) continue;  // no gravity along d: both terms are zero
-      acc[fMOM(d)] += (AT)(G.g[d] * rho_c);
-      acc[fE(ND)] += (AT)(rho_c * (G.g[d] * at(w + (long long)fMOM(d) * N, c)) / (rho_c + rhob_c));
-    }
-  }
-  // ------------------------------------------------------------ update, source, RK, ghosts
-  const double h = A.hfrac * A.dts[0];
-  const OT* __restrict__ base = (const OT*)A.base;
-  OT out[NP];
-#pragma unroll
-  for (int f = 0; f < NP; f++) out[f] = at(base + (long long)f * N, c) + h * (OT)acc[f];
+// The user source and the divB terms of one interior cell (x0, x1, x2) with
+// index c, on its updated values out.
+template <int ND, typename OT>
+__device__ __forceinline__ void add_source(const Geo& G, const RhsArgs& A, unsigned T, int x0, int x1, int x2, unsigned c,
+                                           OT rho_c, OT rhob_c, double h, OT* out) {
+  const long long N = G.N;
+  const int x[3] = {x0, x1, x2};
+  const OT* __restrict__ w = (const OT*)A.win;
+  const OT* __restrict__ bg = (const OT*)A.bg;
   // divB source terms (divb_parallel, src/divb.cu:165-338, 2D), in FP64 on
   // cells 2 < i,j < n-2: divb from the 4th-order differences over 2 p->dx of
   // b + b_b, zeroed on the layers 3, n-4, n-3 (grad3d's mask with interior
@@ -760,141 +348,940 @@ __device__ __forceinline__ void rhs_tile(const Geo& G, const RhsArgs& A, SH* __r
     }
   }
   }
-  if ((T & SMAUG_T_SOURCE) && G.driver == SMAUG_DRIVER_VERTICAL) {
-    const double* dv = G.drv;
-    double ez, exyz;
-    if (A.dshape) {  // separable grid: per-axis factors formed at set-up
-      ez = A.dshape[x[0]];
-      const double exx = A.dshape[G.n[0] + x[1]];
-      exyz = exx * ez;
-      if (ND == 3) exyz = exx * A.dshape[G.n[0] + G.n[1] + x[2]] * ez;
+  // the drivers; spicule1's acts in the step whose counter is 1 only (tdep is
+  // 0 outside it)
+  if (!(T & SMAUG_T_SOURCE) || G.driver == SMAUG_DRIVER_NONE || (G.driver == SMAUG_DRIVER_SPICULE1 && A.tdep == 0.0)) return;
+  const double* dv = G.drv;
+  double ez, exyz;  // the shape: its factor along dim 0, the product of all
+  double xp = 0.0, yp = 0.0;
+  if (G.driver == SMAUG_DRIVER_VERTICAL && A.dshape) {  // separable grid: per-axis factors formed at set-up
+    ez = A.dshape[x[0]];
+    const double exx = A.dshape[G.n[0] + x[1]];
+    exyz = exx * ez;
+    if (ND == 3) exyz = exx * A.dshape[G.n[0] + G.n[1] + x[2]] * ez;
+  } else {
+    double t0, t1, t2 = 0.0;  // exponents along dims 0, 1, 2
+    if (G.driver == SMAUG_DRIVER_SPICULE1) {  // at the grid positions xmin + i dx
+      const double z1 = G.pxmin[0] + (double)x[0] * G.pdx[0] - dv[2];
+      const double x1 = G.pxmin[1] + (double)x[1] * G.pdx[1] - dv[3];
+      t0 = -(z1 * z1) / (dv[5] * dv[5]);
+      t1 = -(x1 * x1) / (dv[6] * dv[6]);
     } else {
       const double zp = at(A.pos, c) - dv[2];
-      const double xp = at(A.pos + N, c) - dv[3];
-      ez = exp(-zp * zp / (dv[5] * dv[5]));
-      const double exx = exp(-xp * xp / (dv[6] * dv[6]));
-      exyz = exx * ez;
+      xp = at(A.pos + N, c) - dv[3];
+      t0 = -zp * zp / (dv[5] * dv[5]);
+      t1 = -xp * xp / (dv[6] * dv[6]);
       if (ND == 3) {
-        const double yp = at(A.pos + 2 * N, c) - dv[4];
-        const double ey = exp(-yp * yp / (dv[6] * dv[6]));
-        exyz = exx * ey * ez;
+        const double wy = G.driver == SMAUG_DRIVER_TORSIONAL ? dv[7] : dv[6];
+        yp = at(A.pos + 2 * N, c) - dv[4];
+        t2 = -yp * yp / (wy * wy);
       }
     }
+    // one exponential in the code, evaluated along dims 1, 2, 0 (exp(0) = 1
+    // for an axis without a factor)
+    exyz = 1.0;
+#pragma unroll 1
+    for (int q = 0; q < 3; q++) {
+      ez = exp(q == 0 ? t1 : (q == 1 ? t2 : t0));
+      exyz = exyz * ez;
+    }
+  }
+  const OT rto = out[fRHO()] + rhob_c;
+  if (G.driver == SMAUG_DRIVER_VERTICAL) {
     // amplitude map: one amplitude per (j,k) column in place of
     // A exp(-dx^2/sxy^2 [- dy^2/sxy^2])
     const OT vz = A.amap ? ((const OT*)A.amap)[x[1] + (ND == 3 ? (long long)G.n[1] * x[2] : 0)] * ez * A.tdep
                          : with_tangent<OT>(dv[0] * exyz * A.tdep, A.damp * exyz * A.tdep);
-    const OT rto = out[fRHO()] + rhob_c;
     out[fMOM(0)] += h * vz * rto;
     out[fE(ND)] += h * (vz * vz) * rto / 2.0;
-  }
-  // fluxtube1's torsional driver (models/usersource.cu.fluxtube1:3-90), 3D
-  if (ND == 3 && (T & SMAUG_T_SOURCE) && G.driver == SMAUG_DRIVER_TORSIONAL) {
-    const double* dv = G.drv;
-    const double xp = at(A.pos + N, c) - dv[3];
-    const double zp = at(A.pos, c) - dv[2];
-    const double yp = at(A.pos + 2 * N, c) - dv[4];
-    const double exz = exp(-zp * zp / (dv[5] * dv[5]));
-    const double exx = exp(-xp * xp / (dv[6] * dv[6]));
-    const double exy = exp(-yp * yp / (dv[7] * dv[7]));
-    const double exyz = exx * exy * exz;
-    const OT vx = with_tangent<OT>((dv[0] * yp / dv[9]) * exyz * A.tdep, (A.damp * yp / dv[9]) * exyz * A.tdep);
-    const OT vy = with_tangent<OT>(-(dv[0] * xp / dv[8]) * exyz * A.tdep, -(A.damp * xp / dv[8]) * exyz * A.tdep);
-    const OT rto = out[fRHO()] + rhob_c;
-    out[fMOM(1)] += h * vx * rto;
-    out[fMOM(2)] += h * vy * rto;
-    out[fE(ND)] += h * (vx * vx + vy * vy) * rto / 2.0;
-  }
-  // spicule1's driver (models/usersource.cu.spicule1:4-136): tdep is 0
-  // outside the step whose counter is 1; grid positions xmin + i dx
-  if ((T & SMAUG_T_SOURCE) && G.driver == SMAUG_DRIVER_SPICULE1 && A.tdep != 0.0) {
-    const double* dv = G.drv;
-    const double xp = G.pxmin[0] + (double)x[0] * G.pdx[0];
-    const double yp = G.pxmin[1] + (double)x[1] * G.pdx[1];
-    const double r1 = (xp - dv[2]) * (xp - dv[2]), r2 = (yp - dv[3]) * (yp - dv[3]);
-    const double g = exp(-r2 / (dv[6] * dv[6])) * exp(-r1 / (dv[5] * dv[5]));
-    const OT vvz = with_tangent<OT>(dv[0] * g * A.tdep, A.damp * g * A.tdep);
-    out[fMOM(0)] = out[fMOM(0)] + h * vvz * (out[fRHO()] + rhob_c);
-  }
-  if (A.r1) {
-#pragma unroll
-    for (int f = 0; f < NP; f++) {
-      const long long o_f = (long long)f * N;
-      out[f] = out[f] + (at((const OT*)A.r1 + o_f, c) + 2.0 * at((const OT*)A.r2 + o_f, c) + at((const OT*)A.r3 + o_f, c) -
-                         4.0 * at(base + o_f, c)) / 3;
+  } else if (G.driver == SMAUG_DRIVER_TORSIONAL) {  // fluxtube1's (models/usersource.cu.fluxtube1:3-90), 3D
+    if constexpr (ND == 3) {
+      const OT vx = with_tangent<OT>((dv[0] * yp / dv[9]) * exyz * A.tdep, (A.damp * yp / dv[9]) * exyz * A.tdep);
+      const OT vy = with_tangent<OT>(-(dv[0] * xp / dv[8]) * exyz * A.tdep, -(A.damp * xp / dv[8]) * exyz * A.tdep);
+      out[fMOM(1)] += h * vx * rto;
+      out[fMOM(2)] += h * vy * rto;
+      out[fE(ND)] += h * (vx * vx + vy * vy) * rto / 2.0;
     }
-  }
-  OT* __restrict__ wo = (OT*)A.wout;
-  // the cell itself, then its ghost images: every combination of its images
-  // across the directions (a fixed direction has none; with n >= 8 an
-  // interior coordinate feeds at most two ghosts per direction), with the
-  // asymm signs.  All indices are compile-time so no register array is
-  // indexed at run time; waves away from the domain edge skip the images.
-#pragma unroll
-  for (int q = 0; q < NP; q++) put(wo + (long long)q * N, c, out[q]);
-  if (!EDGE) return;  // no cell of an inner tile has a ghost image
-#pragma unroll
-  for (int f = 0; f < NP; f++) {
-    if (f > 0 && G.bc_uniform) break;
-    Img2 I[3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-    unsigned neg = 0;  // bit d: direction d flips the sign
-#pragma unroll
-    for (int d = 0; d < ND; d++) {
-      I[d] = bc_images2(G.bct[f][d], x[d], G.n[d], ND);
-      if (G.bct[f][d] == BC_ASYMM) neg |= 1u << d;
-    }
-    if (I[0].m + I[1].m + I[2].m == 0) continue;
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b2 = 0; b2 < 3; b2++)
-#pragma unroll
-        for (int c2 = 0; c2 < (ND == 3 ? 3 : 1); c2++) {
-          if (a + b2 + c2 == 0 || a > I[0].m || b2 > I[1].m || c2 > I[2].m) continue;
-          const int ga = a == 0 ? x[0] : (a == 1 ? I[0].g0 : I[0].g1);
-          const int gb = b2 == 0 ? x[1] : (b2 == 1 ? I[1].g0 : I[1].g1);
-          const int gc = c2 == 0 ? x[2] : (c2 == 1 ? I[2].g0 : I[2].g1);
-          const unsigned cc = cix(G, ga, gb, gc);
-          const unsigned flip = ((a ? 1u : 0u) & neg) ^ ((b2 ? 2u : 0u) & neg) ^ ((c2 ? 4u : 0u) & neg);
-          const bool minus = __builtin_popcount(flip) & 1;
-          if (G.bc_uniform) {
-#pragma unroll
-            for (int q = 0; q < NP; q++) put(wo + (long long)q * N, cc, minus ? -out[q] : out[q]);
-          } else {
-            put(wo + (long long)f * N, cc, minus ? -out[f] : out[f]);
-          }
-        }
+  } else {  // spicule1's (models/usersource.cu.spicule1:4-136)
+    const OT vvz = with_tangent<OT>(dv[0] * exyz * A.tdep, A.damp * exyz * A.tdep);
+    out[fMOM(0)] = out[fMOM(0)] + h * vvz * rto;
   }
 }
 
-// FP32 stencils: at least five wavefronts per SIMD (96 VGPRs; measured
-// faster at 256^3 than four without a spill or six with a 72-byte spill).
-// FP64: three, the number its 52 KB of LDS per workgroup allows (146
-// VGPRs); stating it lets the scheduler spend registers up to that bound
-// (measured 0.8 % faster than a bound of one workgroup).  Dual (the
-// tangent-linear step): its 105 KB of LDS in 3D leave one workgroup per CU
-// whatever the bound, so the compiler may use the accumulation registers
-// too (256 + 10 at gfx950, no scratch); DualF (its mixed-precision form, FP32
-// pairs in 52 KB of LDS): two wavefronts per SIMD.
-template <int ND, typename SH>
-__global__ __launch_bounds__(256, sizeof(SH) == 4 ? 5 : (std::is_same<SH, double>::value ? 3 : 2)) void k_rhs_tiled(Geo G, RhsArgs A) {
-  using L = Lay<ND>;
+// Ghost images of the interior cell x with values out: every combination of
+// its images across the directions (a fixed direction has none; with n >= 8
+// an interior coordinate feeds at most two ghosts per direction), with the
+// asymm signs.  Loops over the combinations (indexed by a number in base 3,
+// a digit per direction: 0 the cell's own coordinate, 1 and 2 its ghosts)
+// and, where the fields' boundary types differ, over the fields, with no
+// register array indexed at run time: the code stays small, as every edge
+// tile streams it.
+template <int ND, typename F>
+__device__ __forceinline__ void each_image(const Geo& G, const int* bct, const int* x, F store) {
+  const int t0 = bct[0], t1 = bct[1], t2 = bct[2];
+  const Img2 I0 = bc_images2(t0, x[0], G.n[0], ND), I1 = bc_images2(t1, x[1], G.n[1], ND);
+  const Img2 I2 = ND == 3 ? bc_images2(t2, x[2], G.n[2], ND) : Img2{0, 0, 0};
+  if (I0.m + I1.m + I2.m == 0) return;
+  const int x0 = x[0], x1 = x[1], x2 = x[2];
+  const int a1 = I0.g0, a2 = I0.g1, b1 = I1.g0, b2 = I1.g1, c1 = I2.g0, c2 = I2.g1;
+#pragma unroll 1
+  for (int q = 1; q < (ND == 3 ? 27 : 9); q++) {
+    const int a = q % 3, b = q / 3 % 3, c = q / 9;
+    if (a > I0.m || b > I1.m || c > I2.m) continue;
+    const unsigned cc = cix(G, a == 0 ? x0 : (a == 1 ? a1 : a2), b == 0 ? x1 : (b == 1 ? b1 : b2),
+                            c == 0 ? x2 : (c == 1 ? c1 : c2));
+    store(cc, ((a && t0 == BC_ASYMM) ^ (b && t1 == BC_ASYMM)) ^ (ND == 3 && c && t2 == BC_ASYMM));
+  }
+}
+template <int ND, typename OT>
+__device__ __forceinline__ void put_images(const Geo& G, OT* __restrict__ wo, const int* x, const OT* out) {
+  constexpr int NP = 2 + 2 * ND;
+  if (G.bc_uniform) {
+    each_image<ND>(G, G.bct[0], x, [&](unsigned cc, bool minus) __attribute__((always_inline)) {
+      // (a pointer per lane, stepped field by field: the bases of all fields
+      // at once would take the scalar registers of the phases' pointers)
+      OT* p = wo + cc;
+#pragma unroll
+      for (int f = 0; f < NP; f++, p += G.N) *p = pick(minus, -out[f], out[f]);
+    });
+  } else {
+#pragma unroll 1
+    for (int f = 0; f < NP; f++) {
+      OT v = out[0];
+#pragma unroll
+      for (int q = 1; q < NP; q++) v = pick(f == q, out[q], v);
+      OT* p = wo + (long long)f * G.N;
+      each_image<ND>(G, G.bct[f], x, [&](unsigned cc, bool minus) __attribute__((always_inline)) { put(p, cc, pick(minus, -v, v)); });
+    }
+  }
+}
+
+// The terms of one tile whose origin (first interior cell) is o.  EDGE
+// false: every cell of the tile lies in [5, n-6] along every direction, so
+// no cell of it or of its halos is a ghost or on a zeroed layer, every
+// staged box lies inside the grid and no cell has a ghost image; the
+// boundary checks are then compiled out (the arithmetic is the same).
+// SEP: the grid is a tensor product (A.dx1 set).
+// ALL: every direction's fluxes, every q box and the products of a group of
+// phases have their own place in LDS, so the phases need 6 barriers and 3
+// trips to memory where the others take 20 and 11 (see k_rhs_small).
+template <class TL, typename SH, bool EDGE, bool SEP, bool ALL>
+__device__ __forceinline__ void rhs_tile(const Geo& G, const RhsArgs& A, SH* __restrict__ sm, const int* o) {
+  using L = Lay<TL>;
+  using AT = SH;                        // arithmetic type of the stencils
+  using V = typename ValT<SH>::T;       // its values (coefficients carry no tangent)
+  // own-cell type: FP64 (the own-cell update and the RK combination are
+  // FP64 with FP32 stencils too), Dual in the tangent-linear step
+  using OT = typename OwnT<SH>::T;
+  constexpr int ND = L::ND, XC = L::XC, NP = L::NP;
   constexpr int TX = L::TX, TY = L::TY, TZ = L::TZ;
-  __shared__ SH sm[L::SMEM];
   const int tid = threadIdx.x;
-  if (A.zero_next && blockIdx.x == 0 && tid < 3) A.zero_next[tid] = 0ull;
-  // XCD-aware tile order: the hardware deals consecutive workgroups to the
-  // 8 XCDs in turn, so workgroup b runs on XCD b%8.  In 3D XCD x takes the
-  // slab of tile layers [x*gz/8, (x+1)*gz/8) and walks it x fastest, then
-  // z, then y, so the z neighbour of a tile runs gx tiles after it (its
-  // halo planes still in that XCD's L2) and the y neighbour gx*gz/8 tiles
-  // after it (measured 1.7 % faster at 256^3 than x, y, z order, whose z
-  // neighbour comes gx*gy tiles later); otherwise XCD x takes the tiles
-  // [x*nb/8, (x+1)*nb/8) in x, y, z order.
+  const int lc[3] = {tid % (TX / XC) * XC, (tid / (TX / XC)) % TY, ND == 3 ? tid / (TX / XC * TY) : 0};
+  const int x[3] = {o[0] + lc[0], o[1] + lc[1], o[2] + lc[2]};  // first cell of the thread
+  bool valid[XC], any = false;
+#pragma unroll
+  for (int u = 0; u < XC; u++) {
+    const int y[3] = {x[0] + u, x[1], x[2]};
+    valid[u] = !EDGE || interior_c<ND>(G, y);
+    any = any || valid[u];
+  }
+  const long long N = G.N;
+  const unsigned c = cix(G, x[0], x[1], x[2]);  // own cell (used by valid threads only)
+  const OT* __restrict__ w = (const OT*)A.win;    // own-cell values
+  const SH* __restrict__ ws = (const SH*)A.wsh;    // neighbour values (stencil precision)
+  const OT* __restrict__ bg = (const OT*)A.bg;  // background (Dual in the tangent-linear step)
+  const SH* __restrict__ pr = (const SH*)A.prim;
+  const unsigned T = G.terms;
+  AT acc[NP][XC];
+#pragma unroll
+  for (int f = 0; f < NP; f++)
+#pragma unroll
+    for (int u = 0; u < XC; u++) acc[f][u] = AT(0);
+
+  auto pin_acc = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int f = 0; f < NP; f++)
+#pragma unroll
+      for (int u = 0; u < XC; u++) pin(acc[f][u]);
+  };
+
+  V* const SDX = reinterpret_cast<V*>(sm + (ALL ? L::DXO_ALL : L::DXO));  // spacing table (tensor-product grids)
+  if (SEP && tid < L::DXT) {  // visible after the first barrier
+    const int n0 = G.n[0], n1 = G.n[1], n2 = ND == 3 ? G.n[2] : 0, o0 = o[0], o1 = o[1], o2 = o[2];
+    const bool d0 = tid < TX, d1 = tid < TX + TY;
+    const int xx = d0 ? o0 + tid : (d1 ? o1 + tid - TX : o2 + tid - TX - TY);
+    const int od = d0 ? 0 : (d1 ? n0 : n0 + n1);
+    const bool ing = xx < (d0 ? n0 : (d1 ? n1 : n2));
+    SDX[tid] = ing ? (V)A.dx1[od + xx] : V(1);
+    SDX[L::DXT + tid] = ing ? (V)A.rdx1[od + xx] : V(1);
+  }
+  // delx and 1/delx along d at the thread's cells
+  auto dxs = [&](int d, V* dx) __attribute__((always_inline)) {
+    const int t = d == 0 ? lc[0] : (d == 1 ? TX + lc[1] : TX + TY + lc[2]);
+#pragma unroll
+    for (int u = 0; u < XC; u++)
+      dx[u] = SEP ? SDX[t + (d == 0 ? u : 0)] : (valid[u] ? (V)at(A.delx + (long long)d * N, c + u) : V(1));
+  };
+  auto rdxs = [&](int d, V* rdx) __attribute__((always_inline)) {
+    const int t = L::DXT + (d == 0 ? lc[0] : (d == 1 ? TX + lc[1] : TX + TY + lc[2]));
+#pragma unroll
+    for (int u = 0; u < XC; u++)
+      rdx[u] = SEP ? SDX[t + (d == 0 ? u : 0)] : (valid[u] ? (V)at(A.rdelx + (long long)d * N, c + u) : V(1));
+  };
+  // XC values of an own-cell array (0 where the cell is not interior); the
+  // index is pinned, so values that several phases read come from the cache
+  // again and do not occupy registers between them
+  auto own = [&](const auto* __restrict__ p, auto* v) __attribute__((always_inline)) {
+    using E = std::remove_reference_t<decltype(v[0])>;
+    unsigned cc = c;
+    pin(cc);
+    if (!EDGE || valid[XC - 1]) {  // the tile starts on an interior cell: the last one valid means all are
+      ldg<XC>(p, cc, v);
+    } else {
+#pragma unroll
+      for (int u = 0; u < XC; u++) v[u] = valid[u] ? at(p, cc + u) : E(0);
+    }
+  };
+
+  const bool want_mom = G.hyper && (T & SMAUG_T_HMOM);
+  const bool want_eterm = (T & SMAUG_T_ETERM) != 0;
+  const bool want_b = G.hyper && (T & SMAUG_T_HB);
+
+  // ------------------------------------------------------------ fluxes
+  if (T & SMAUG_T_FLUX) {
+    // the thread's own cells: their state is loaded once for every
+    // direction; a second slot per direction covers the 2 + 2 halo layers
+    // along it, its state loaded while the direction before it is summed
+    CellState<ND, AT> S0[XC], S1;
+    bool in0[XC];
+    auto FB = [&](int d) __attribute__((always_inline)) { return sm + (ALL ? d * L::FLX : 0); };
+#pragma unroll
+    for (int u = 0; u < XC; u++) {
+      const int y[3] = {x[0] + u, x[1], x[2]};
+      in0[u] = !EDGE || in_grid<ND>(G, y);
+    }
+    if (in0[XC - 1]) {
+      load_cells<ND, XC, SH, AT>(G, ws, bg, c, S0);
+    } else {
+#pragma unroll
+      for (int u = 0; u < XC; u++)
+        if (in0[u]) load_cell<ND, SH, AT>(G, ws, bg, c + u, S0[u]);
+    }
+    bool in1 = false;
+    int l1 = 0;
+    // halo slot of direction d: its state (or out of the grid) and its place
+    auto halo = [&](int d) __attribute__((always_inline)) {
+      const int ex[3] = {d == 0 ? 2 : 0, d == 1 ? 2 : 0, d == 2 ? 2 : 0};
+      const int rx = TX + 2 * ex[0], ry = TY + 2 * ex[1];
+      const int Td = d == 0 ? TX : (d == 1 ? TY : TZ);
+      const int pa = d == 0 ? 1 : 0, qa = d == 2 ? 1 : 2;  // the other two axes
+      const int Tp = pa == 0 ? TX : TY;
+      const int Fd = Tp * (ND == 3 ? (qa == 1 ? TY : TZ) : 1);  // face of the tile across d
+      in1 = false;
+      l1 = -1;
+      if (tid < 4 * Fd) {
+        // along dim 0 the two layers of a side follow each other, so the
+        // lanes of a wavefront read neighbouring cells
+        const int layer = d == 0 ? tid % 2 + 2 * (tid / (2 * Fd)) : tid / Fd;
+        const int r = d == 0 ? tid % (2 * Fd) / 2 : tid - layer * Fd;
+        int rc[3] = {0, 0, 0};
+        rc[d] = layer < 2 ? layer : Td + layer;  // region coordinates 0, 1 and Td+2, Td+3
+        rc[pa] = r % Tp;
+        if (ND == 3) rc[qa] = r / Tp;
+        const int xr[3] = {o[0] - ex[0] + rc[0], o[1] - ex[1] + rc[1], ND == 3 ? o[2] - ex[2] + rc[2] : 0};
+        in1 = !EDGE || in_grid<ND>(G, xr);
+        l1 = rc[0] + rx * (rc[1] + ry * rc[2]);
+        if (in1) load_cell<ND, SH, AT>(G, ws, bg, cix(G, xr[0], xr[1], xr[2]), S1);
+      }
+    };
+    static_assert(ND == 3 ? 4 * TY * TZ <= L::NT && 4 * TX * TZ <= L::NT && 4 * TX * TY <= L::NT
+                          : 4 * TX <= L::NT && 4 * TY <= L::NT,
+                  "the halo layers of a direction fit one slot per thread");
+    // the fluxes along d of the own cells and the halo slot to LDS
+    auto form = [&](int d) __attribute__((always_inline)) {
+      const int ex[3] = {d == 0 ? 2 : 0, d == 1 ? 2 : 0, d == 2 ? 2 : 0};
+      const int rx = TX + 2 * ex[0], ry = TY + 2 * ex[1];
+      // slot of field f (the flux of b_d along d is zero: not kept)
+      auto slot = [&](int f) __attribute__((always_inline)) { return (f < fB(ND, d) ? f : f - 1) * L::FN; };
+      const int l0 = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
+      {
+        AT F[XC][NP];
+#pragma unroll
+        for (int u = 0; u < XC; u++) {
+          if (in0[u]) {
+            pin(S0[u]);
+            fluxes_of<ND, AT>(G, S0[u], d, F[u]);
+          } else {
+#pragma unroll
+            for (int f = 0; f < NP; f++) F[u][f] = AT(0);
+          }
+        }
+#pragma unroll
+        for (int f = 0; f < NP; f++) {
+          if (f == fB(ND, d)) continue;
+          AT p[XC];
+#pragma unroll
+          for (int u = 0; u < XC; u++) p[u] = F[u][f];
+          stl<XC>(FB(d) + slot(f) + l0, p);
+        }
+      }
+      if (l1 >= 0) {
+        AT F[NP];
+        if (in1) {
+          fluxes_of<ND, AT>(G, S1, d, F);
+        } else {
+#pragma unroll
+          for (int f = 0; f < NP; f++) F[f] = AT(0);
+        }
+#pragma unroll
+        for (int f = 0; f < NP; f++)
+          if (f != fB(ND, d)) FB(d)[slot(f) + l1] = F[f];
+      }
+    };
+    // their divergence
+    auto diverge = [&](int d) __attribute__((always_inline)) {
+      const int ex[3] = {d == 0 ? 2 : 0, d == 1 ? 2 : 0, d == 2 ? 2 : 0};
+      const int rx = TX + 2 * ex[0], ry = TY + 2 * ex[1];
+      // slot of field f (the flux of b_d along d is zero: not kept)
+      auto slot = [&](int f) __attribute__((always_inline)) { return (f < fB(ND, d) ? f : f - 1) * L::FN; };
+      const int l0 = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
+      V inv[XC];
+      rdxs(d, inv);
+      bool z[XC];
+#pragma unroll
+      for (int u = 0; u < XC; u++) {
+        inv[u] *= V(1.0 / 12.0);
+        z[u] = !valid[u] || z4e<EDGE>(G, zFLUX(ND), d, x[d] + (d == 0 ? u : 0));
+      }
+      const int s = d == 0 ? 1 : (d == 1 ? rx : rx * ry);
+#pragma unroll
+      for (int f = 0; f < NP; f++) {
+        if (f == fB(ND, d)) continue;
+        const AT* Fp = FB(d) + slot(f) + l0;
+        AT a[XC], b[XC], e[XC], g[XC];  // F at i-2, i-1, i+1, i+2
+        if (d == 0 && XC == 2) {
+          AT m[XC], p[XC], q[XC];
+          ldl<XC>(Fp - 2, m);
+          ldl<XC>(Fp, p);
+          ldl<XC>(Fp + 2, q);
+          a[0] = m[0];
+          b[0] = a[XC - 1] = m[XC - 1];
+          b[XC - 1] = p[0];
+          e[0] = p[XC - 1];
+          g[0] = e[XC - 1] = q[0];
+          g[XC - 1] = q[XC - 1];
+        } else {
+          ldl<XC>(Fp - 2 * s, a);
+          ldl<XC>(Fp - s, b);
+          ldl<XC>(Fp + s, e);
+          ldl<XC>(Fp + 2 * s, g);
+        }
+#pragma unroll
+        for (int u = 0; u < XC; u++)
+          acc[f][u] -= z[u] ? AT(0) : ((V(8) * e[u] - V(8) * b[u]) + (a[u] - g[u])) * inv[u];
+      }
+      pin_acc();
+    };
+    halo(0);
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+      form(d);
+      if (d + 1 < ND) halo(d + 1);
+      if (!ALL) {
+        __syncthreads();
+        diverge(d);
+        __syncthreads();
+      }
+    }
+    if (ALL) {
+      __syncthreads();
+#pragma unroll
+      for (int d = 0; d < ND; d++) diverge(d);
+      __syncthreads();
+    }
+  } else if (SEP) {
+    __syncthreads();  // the spacing table
+  }
+
+  // ------------------------------------------------------------ hyperdiffusion + energy terms
+  SH* const CBX = sm;                                  // rho_t (tile + 1)
+  // q box i (ALL: rho, q_e, v_f, b_f; else the one of the phase), region
+  // arrays of phase f: products of the cross directions, energy
+  auto QB = [&](int i) __attribute__((always_inline)) { return sm + L::PN + (ALL ? i * L::QN : 0); };
+  auto NRF = [&](int f) __attribute__((always_inline)) { return sm + L::PN + (ALL ? NP * L::QN + f * ND * L::RN : L::QN); };
+  constexpr int QV = 2, QM = 2 + ND;  // boxes of v_0 and b_0
+  // tile-cell index in the q box and its strides
+  const int qc = (lc[0] + L::HX) + L::QX * ((lc[1] + 3) + L::QY * (ND == 3 ? lc[2] + 3 : 0));
+  const int qs[3] = {1, L::QX, L::QX * L::QY};
+  const int pc = (lc[0] + L::RX) + L::PX * ((lc[1] + 1) + L::PY * (ND == 3 ? lc[2] + 1 : 0));
+  const int ps[3] = {1, L::PX, L::PX * L::PY};
+
+  V cm[ND];
+#pragma unroll
+  for (int d = 0; d < ND; d++) cm[d] = (V)__longlong_as_double((long long)A.cmax_bits[d]);
+  auto scales = [&](int d, V k, V* sc) __attribute__((always_inline)) {
+    dxs(d, sc);
+#pragma unroll
+    for (int u = 0; u < XC; u++) sc[u] *= cm[d] * k;
+  };
+
+  const bool mom_phases = want_mom || want_eterm;
+  QBox<TL, SH, EDGE> Q;  // the next q box on its way
+
+  // rho (src/hyperdifrhosource1.cu) and e_int (src/hyperdifesource1.cu):
+  // both boxes are staged in one round trip (ahead of the rho_t box's use)
+  const bool h_rho = G.hyper && (T & SMAUG_T_HRHO), h_e = G.hyper && (T & SMAUG_T_HE);
+  const SH* qe = pr + (long long)pQE(ND) * N;
+  SH* const box_rho = ALL ? QB(0) : sm;
+  SH* const box_e = ALL ? QB(1) : sm + L::QN;
+  if (ALL) {  // every box that a phase will read
+    auto src = [&](int i) __attribute__((always_inline)) {
+      return i == 0 ? ws : (i == 1 ? qe : (i < QM ? pr + (long long)pV(i - QV) * N : ws + (long long)fB(ND, i - QM) * N));
+    };
+    if constexpr (EDGE) {
+      constexpr int NE = (L::QN + L::NT - 1) / L::NT;
+      int from[NE];
+#pragma unroll
+      for (int k = 0; k < NE; k++) {
+        const int l = imin(tid + L::NT * k, L::QN - 1);
+        const int a = l % L::QX, b = (l / L::QX) % L::QY, e = l / (L::QX * L::QY);
+        from[k] = q_source<ND>(G, o[0] - L::HX + a, o[1] - 3 + b, ND == 3 ? o[2] - 3 + e : 0);
+      }
+      SH v[NP][NE];
+#pragma unroll
+      for (int i = 0; i < NP; i++)
+#pragma unroll
+        for (int k = 0; k < NE; k++) v[i][k] = from[k] >= 0 ? at(src(i), (unsigned)from[k]) : SH(0);
+      if (want_mom) stage_rho_t<TL, SH, EDGE>(G, ws, bg, CBX, o);
+#pragma unroll
+      for (int i = 0; i < NP; i++)
+#pragma unroll
+        for (int k = 0; k < NE; k++)
+          if (tid + L::NT * k < L::QN) QB(i)[tid + L::NT * k] = v[i][k];
+    } else {
+      QBox<TL, SH, EDGE> B[NP];
+#pragma unroll
+      for (int i = 0; i < NP; i++) B[i].load(G, src(i), o);
+      if (want_mom) stage_rho_t<TL, SH, EDGE>(G, ws, bg, CBX, o);
+#pragma unroll
+      for (int i = 0; i < NP; i++) B[i].store(G, src(i), QB(i), o);
+    }
+    __syncthreads();
+  }
+  if (h_rho || h_e) {
+    if (!ALL) {
+    __builtin_amdgcn_s_setprio(3);
+    if (h_rho && h_e) {
+      QBox<TL, SH, EDGE> Q2;
+      Q.load(G, ws, o);
+      Q2.load(G, qe, o);
+      __builtin_amdgcn_s_setprio(0);
+      Q.store(G, ws, box_rho, o);
+      Q2.store(G, qe, box_e, o);
+    } else {
+      const SH* qa = h_rho ? ws : qe;
+      Q.load(G, qa, o);
+      __builtin_amdgcn_s_setprio(0);
+      Q.store(G, qa, h_rho ? box_rho : box_e, o);
+    }
+    __syncthreads();
+    }
+    auto diffuse = [&](const SH* box, int f, int zidx) __attribute__((always_inline)) {
+#pragma unroll
+      for (int d = 0; d < ND; d++) {
+        V sc[XC], rdx[XC];
+        scales(d, (V)G.chyp[f], sc);
+        rdxs(d, rdx);
+        Win<TL, SH> W;
+        if (d == 0) W.template load<0>(box, qc, 1, sc);
+        else W.template load<1>(box, qc, qs[d], sc);
+#pragma unroll
+        for (int u = 0; u < XC; u++) {
+          const bool z = !valid[u] || z1e<EDGE>(G, zidx, d, x[d] + (d == 0 ? u : 0));
+          const AT gr = z ? AT(0) : (W.q[u][3] - W.q[u][2]) * rdx[u];
+          const AT gl = z ? AT(0) : (W.q[u][2] - W.q[u][1]) * rdx[u];
+          acc[f][u] += (gr * W.nr[u] - gl * W.nl[u]) * rdx[u];
+          pin(acc[f][u]);
+        }
+      }
+    };
+    if (h_rho) diffuse(box_rho, fRHO(), zRHO);
+    if (h_e) diffuse(box_e, fE(ND), zTMP1);
+    if (!ALL) __syncthreads();
+  }
+
+  // momentum phases (q = v_f): energy terms, diagonal and off-diagonal
+  // sources; then magnetic phases (q = b_f).  A phase has two parts with a
+  // barrier between them: the windows of the q box (coefficients, diagonal
+  // terms, and the cross products of the tile extended by one layer along
+  // f), then the differences of the products along f, during which the next
+  // phase's q box travels.
+  // Products of phase f at the tile's region: cross direction k in NR + k RN,
+  // their energy terms summed in NR + (ND-1) RN.
+  auto region = [&](int f, int& rx, int& ry, int* ex) __attribute__((always_inline)) {
+    ex[0] = f == 0 ? L::RX : 0;
+    ex[1] = f == 1 ? 1 : 0;
+    ex[2] = f == 2 ? 1 : 0;
+    rx = TX + 2 * ex[0];
+    ry = TY + 2 * ex[1];
+  };
+  // the two layers just outside the tile along f: one (cell, cross
+  // direction) per thread; the directions of a cell sit in lanes l and l^32
+  // of a wavefront, which add up their energy products
+  auto border = [&](int f, const SH* qb, AT* NR, V Kc, int zidx, int m0, bool weigh, V fac) __attribute__((always_inline)) {
+    int rx, ry, ex[3];
+    region(f, rx, ry, ex);
+    const int pd = f == 0 ? 1 : 0, qd = f == 2 ? 1 : 2;
+    const int Tp = pd == 0 ? TX : TY, Tq = ND == 3 ? (qd == 1 ? TY : TZ) : 1;
+    const int Fc = Tp * Tq;
+    const int ntask = 2 * Fc * (ND - 1);
+    const int k = ND == 3 ? (tid >> 5) & 1 : 0;                      // cross direction
+    const int r2 = ND == 3 ? (tid & 31) + 32 * (tid >> 6) : tid;     // border cell
+    AT gp = AT(0), ge = AT(0);
+    int l = 0;
+    if (tid < ntask) {
+      const int side = r2 >= Fc ? 1 : 0, r = r2 - side * Fc;
+      int bc[3] = {0, 0, 0};
+      bc[f] = side ? (f == 0 ? TX : (f == 1 ? TY : TZ)) : -1;
+      bc[pd] = r % Tp;
+      if (ND == 3) bc[qd] = r / Tp;
+      l = (bc[0] + ex[0]) + rx * ((bc[1] + ex[1]) + ry * (bc[2] + ex[2]));
+      const int xr[3] = {o[0] + bc[0], o[1] + bc[1], ND == 3 ? o[2] + bc[2] : 0};
+      if (!EDGE || interior_c<ND>(G, xr)) {
+        const unsigned gq = cix(G, xr[0], xr[1], xr[2]);
+        // d != f: the border cell's coordinate along d is a tile coordinate
+        const bool kk = ND == 3 && k;
+        const int bp = bc[pd], bq = bc[qd], xp = xr[pd], xq = xr[qd], sp = qs[pd], sq = qs[qd];
+        const SH* mp = ws + (long long)(m0 + pd) * N;
+        const SH* mq = ws + (long long)(m0 + qd) * N;
+        const AT mb = at(kk ? mq : mp, gq);
+        const int qi = (bc[0] + L::HX) + L::QX * ((bc[1] + 3) + L::QY * (ND == 3 ? bc[2] + 3 : 0));
+        const int s = kk ? sq : sp;
+        const int tp = (pd == 0 ? 0 : TX) + bp, tq = (qd == 1 ? TX : TX + TY) + bq;
+        const int ti = kk ? tq : tp;
+        const V cp = cm[pd], cq = cm[ND == 3 ? qd : 0];
+        const V cmd = kk ? cq : cp;
+        // (edge tiles of FP32 dual numbers read the spacing arrays here: with
+        // the table the compiler reserves 68 bytes of scratch that no
+        // instruction touches)
+        constexpr bool table = SEP && !(EDGE && ND == 3 && std::is_same<SH, DualF>::value);
+        const V dxr = table ? SDX[ti] : (V)at(A.delx + (long long)(kk ? qd : pd) * N, gq);
+        const V rdxr = table ? SDX[L::DXT + ti] : (V)at(A.rdelx + (long long)(kk ? qd : pd) * N, gq);
+        const bool z = kk ? z1e<EDGE>(G, zidx, qd, xq) : z1e<EDGE>(G, zidx, pd, xp);
+        SH w7[7];
+        V y[7], R[2];
+#pragma unroll
+        for (int q = 0; q < 7; q++) {
+          w7[q] = qb[qi + (q - 3) * s];
+          y[q] = valof(w7[q]);
+        }
+        nu_ratios<2>(y, R);
+        const AT t5 = z ? AT(0) : (w7[4] - w7[2]) * rdxr * V(0.5);
+        const AT t6 = t5 * (dxr * cmd * Kc * (R[1] + R[0])) * fac;
+        ge = t6 * mb;
+        gp = weigh ? CBX[(bc[0] + L::RX) + L::PX * ((bc[1] + 1) + L::PY * (ND == 3 ? bc[2] + 1 : 0))] * t6 : t6;
+      }
+    }
+    if (ND == 3) ge = ge + lane_xor32(ge);
+    if (tid < ntask) {
+      NR[(ND == 3 ? k : 0) * L::RN + l] = gp;
+      if (k == 0) NR[(ND - 1) * L::RN + l] = ge;
+    }
+  };
+
+  if (mom_phases) {
+    if (!ALL) {
+      Q.load(G, pr + (long long)pV(0) * N, o);
+      if (want_mom) stage_rho_t<TL, SH, EDGE>(G, ws, bg, CBX, o);
+      Q.store(G, pr + (long long)pV(0) * N, QB(QV), o);
+    }
+    AT ptb[XC], bb[ND][XC];  // background terms of the energy source, formed in FP64
+    if (want_eterm) {
+      OT eb[XC], bb2[XC];
+      own(bg + (long long)bEB() * N, eb);
+#pragma unroll
+      for (int d = 0; d < ND; d++) {
+        OT b1[XC];
+        own(bg + (long long)bBB(d) * N, b1);
+#pragma unroll
+        for (int u = 0; u < XC; u++) {
+          bb2[u] = d == 0 ? b1[u] * b1[u] : bb2[u] + b1[u] * b1[u];
+          bb[d][u] = (AT)b1[u];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < XC; u++) ptb[u] = (AT)((G.gamma - 1) * eb[u] - 0.5 * (G.gamma - 2) * bb2[u]);
+    }
+    AT mo[ND][XC];  // own momenta
+    if (want_mom)
+#pragma unroll
+      for (int d = 0; d < ND; d++) own(ws + (long long)fMOM(d) * N, mo[d]);
+    if (!ALL) __syncthreads();
+    auto part1 = [&](int f) __attribute__((always_inline)) {
+      const SH* qb = QB(QV + f);
+      AT* NR = NRF(f);
+      int rx, ry, ex[3];
+      region(f, rx, ry, ex);
+      const int ri = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
+      const V Kc = (V)G.chyp[fMOM(f)];
+      AT ge[XC], rt[XC];
+#pragma unroll
+      for (int u = 0; u < XC; u++) ge[u] = AT(0);
+      if (want_mom) ldl<XC>(CBX + pc, rt);
+#pragma unroll
+      for (int d = 0; d < ND; d++) {
+        V sc[XC], rdx[XC];
+        scales(d, Kc, sc);
+        rdxs(d, rdx);
+        Win<TL, SH> W;
+        if (d == 0) W.template load<0>(qb, qc, 1, sc);
+        else W.template load<1>(qb, qc, qs[d], sc);
+        if (want_eterm) {  // addenergyterms_cd2 for dir f
+#pragma unroll
+          for (int u = 0; u < XC; u++) {
+            const AT g4 = !valid[u] || z4e<EDGE>(G, zVEL(f), d, x[d] + (d == 0 ? u : 0))
+                              ? AT(0)
+                              : ((V(8) * W.q[u][3] - V(8) * W.q[u][1]) + (W.q[u][0] - W.q[u][4])) * (rdx[u] * V(1.0 / 12.0));
+            acc[fE(ND)][u] += d == f ? (bb[f][u] * bb[f][u] - ptb[u]) * g4 : bb[d][u] * bb[f][u] * g4;
+          }
+        }
+        if (want_mom) {
+          // diagonal source along d, and the products rho_t*t6, t6*m_d of
+          // the cross direction d (src/hyperdifmomsource1.cu,
+          // src/hyperdifmomsourcene1.cu); m_f at the faces from rho_t v_f
+          AT rp[XC], rm[XC];
+          if (d == 0 && XC == 2) {
+            AT a[XC], b[XC];
+            ldl<XC>(CBX + pc - 2, a);
+            ldl<XC>(CBX + pc + 2, b);
+            rm[0] = a[XC - 1];
+            rm[XC - 1] = rt[0];
+            rp[0] = rt[XC - 1];
+            rp[XC - 1] = b[0];
+          } else {
+            ldl<XC>(CBX + pc + ps[d], rp);
+            ldl<XC>(CBX + pc - ps[d], rm);
+          }
+          AT gp[XC];
+#pragma unroll
+          for (int u = 0; u < XC; u++) {
+            const bool z = !valid[u] || z1e<EDGE>(G, zTMP4, d, x[d] + (d == 0 ? u : 0));
+            const AT q0 = W.q[u][2], qp = W.q[u][3], qm = W.q[u][1];
+            const V hr = rdx[u] * V(0.5);
+            const V wd = d == f ? hr : hr * V(0.5);  // (the face averages' 1/2; d == f counts twice)
+            const AT gr = z ? AT(0) : (qp - q0) * (W.nr[u] * rdx[u]);
+            const AT gl = z ? AT(0) : (q0 - qm) * (W.nl[u] * rdx[u]);
+            const AT m0 = rt[u] * q0;
+            acc[fMOM(f)][u] += ((rt[u] + rp[u]) * gr - (rt[u] + rm[u]) * gl) * wd;
+            acc[fE(ND)][u] += ((m0 + rp[u] * qp) * gr - (m0 + rm[u] * qm) * gl) * wd;
+            if (d != f) {
+              const AT t6 = z ? AT(0) : (qp - qm) * ((W.nr[u] + W.nl[u]) * (hr * V(0.25)));
+              gp[u] = rt[u] * t6;
+              ge[u] += t6 * mo[d][u];
+            }
+          }
+          if (d != f) stl<XC>(NR + (d < f ? d : d - 1) * L::RN + ri, gp);
+        }
+        pin_acc();
+      }
+      if (want_mom) {
+        stl<XC>(NR + (ND - 1) * L::RN + ri, ge);
+        border(f, qb, NR, Kc, zTMP4, fMOM(0), true, V(0.25));
+      }
+    };
+    auto part2 = [&](int f) __attribute__((always_inline)) {
+      if (want_mom) {
+        const AT* NR = NRF(f);
+        int rx, ry, ex[3];
+        region(f, rx, ry, ex);
+        const int sf = f == 0 ? 1 : (f == 1 ? rx : rx * ry);
+        const int ri = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
+        V rdx[XC];
+        rdxs(f, rdx);
+        AT dif[ND][XC];
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+          AT p[XC], m[XC];
+          const AT* R = NR + k * L::RN + ri;
+          if (f == 0 && XC == 2) {
+            AT a[XC], b[XC], e[XC];
+            ldl<XC>(R - 2, a);
+            ldl<XC>(R, b);
+            ldl<XC>(R + 2, e);
+            m[0] = a[XC - 1];
+            p[0] = b[XC - 1];
+            m[XC - 1] = b[0];
+            p[XC - 1] = e[0];
+          } else {
+            ldl<XC>(R + sf, p);
+            ldl<XC>(R - sf, m);
+          }
+#pragma unroll
+          for (int u = 0; u < XC; u++) {
+            const bool z = !valid[u] || z1e<EDGE>(G, k == ND - 1 ? zTMP8 : zTMP7, f, x[f] + (f == 0 ? u : 0));
+            dif[k][u] = z ? AT(0) : (p[u] - m[u]) * (rdx[u] * V(0.5));
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < XC; u++) {
+#pragma unroll
+          for (int d = 0; d < ND; d++)
+            if (d != f) acc[fMOM(d)][u] += dif[d < f ? d : d - 1][u];
+          acc[fE(ND)][u] += dif[ND - 1][u];
+        }
+        pin_acc();
+      }
+    };
+#pragma unroll
+    for (int f = 0; f < ND; f++) {
+      part1(f);
+      if (!ALL) {
+        __syncthreads();
+        const bool more = f + 1 < ND;
+        const SH* nq = pr + (long long)pV(more ? f + 1 : 0) * N;
+        if (more) Q.load(G, nq, o);
+        part2(f);
+        if (more) {
+          Q.store(G, nq, QB(QV), o);
+          __syncthreads();
+        }
+      }
+    }
+    if (ALL) {
+      __syncthreads();
+#pragma unroll
+      for (int f = 0; f < ND; f++) part2(f);
+      __syncthreads();
+    }
+  }
+
+  // magnetic phases (q = b_f): curl-form cross terms (sb = -1,
+  // src/hyperdifbsourcene1.cu) and diagonal terms (sb = +1,
+  // src/hyperdifbsource1.cu)
+  if (want_b) {
+    if (!ALL) {
+      Q.load(G, ws + (long long)fB(ND, 0) * N, o);
+      Q.store(G, ws + (long long)fB(ND, 0) * N, QB(QM), o);
+    }
+    AT bo[ND][XC];  // own field
+#pragma unroll
+    for (int d = 0; d < ND; d++) own(ws + (long long)fB(ND, d) * N, bo[d]);
+    if (!ALL) __syncthreads();
+    auto part1 = [&](int f) __attribute__((always_inline)) {
+      const SH* qb = QB(QM + f);
+      AT* NR = NRF(f);
+      int rx, ry, ex[3];
+      region(f, rx, ry, ex);
+      const int ri = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
+      const V Kc = (V)G.chyp[fB(ND, f)];
+      AT ge[XC];
+#pragma unroll
+      for (int u = 0; u < XC; u++) ge[u] = AT(0);
+#pragma unroll
+      for (int d = 0; d < ND; d++) {
+        if (d == f) continue;
+        V sc[XC], rdx[XC];
+        scales(d, Kc, sc);
+        rdxs(d, rdx);
+        Win<TL, SH> W;
+        if (d == 0) W.template load<0>(qb, qc, 1, sc);
+        else W.template load<1>(qb, qc, qs[d], sc);
+        AT gp[XC];
+#pragma unroll
+        for (int u = 0; u < XC; u++) {
+          const bool z = !valid[u] || z1e<EDGE>(G, zTMP1, d, x[d] + (d == 0 ? u : 0));
+          const AT q0 = W.q[u][2], qp = W.q[u][3], qm = W.q[u][1];
+          const AT gr = z ? AT(0) : (qp - q0) * (W.nr[u] * rdx[u]);
+          const AT gl = z ? AT(0) : (q0 - qm) * (W.nl[u] * rdx[u]);
+          acc[fB(ND, f)][u] += (gr - gl) * rdx[u];
+          acc[fE(ND)][u] += ((q0 + qp) * gr - (q0 + qm) * gl) * (rdx[u] * V(0.5));
+          gp[u] = z ? AT(0) : (qp - qm) * ((W.nr[u] + W.nl[u]) * (rdx[u] * V(0.25)));
+          ge[u] += gp[u] * bo[d][u];
+        }
+        stl<XC>(NR + (d < f ? d : d - 1) * L::RN + ri, gp);
+        pin_acc();
+      }
+      stl<XC>(NR + (ND - 1) * L::RN + ri, ge);
+      border(f, qb, NR, Kc, zTMP1, fB(ND, 0), false, V(0.5));
+    };
+    auto part2 = [&](int f) __attribute__((always_inline)) {
+      const AT* NR = NRF(f);
+      int rx, ry, ex[3];
+      region(f, rx, ry, ex);
+      const int sf = f == 0 ? 1 : (f == 1 ? rx : rx * ry);
+      const int ri = (lc[0] + ex[0]) + rx * ((lc[1] + ex[1]) + ry * (lc[2] + ex[2]));
+      V rdx[XC];
+      rdxs(f, rdx);
+#pragma unroll
+      for (int k = 0; k < ND; k++) {
+        AT p[XC], m[XC];
+        const AT* R = NR + k * L::RN + ri;
+        if (f == 0 && XC == 2) {
+          AT a[XC], b[XC], e[XC];
+          ldl<XC>(R - 2, a);
+          ldl<XC>(R, b);
+          ldl<XC>(R + 2, e);
+          m[0] = a[XC - 1];
+          p[0] = b[XC - 1];
+          m[XC - 1] = b[0];
+          p[XC - 1] = e[0];
+        } else {
+          ldl<XC>(R + sf, p);
+          ldl<XC>(R - sf, m);
+        }
+#pragma unroll
+        for (int u = 0; u < XC; u++) {
+          const bool z = !valid[u] || z1e<EDGE>(G, k == ND - 1 ? zTMP5 : zTMP3, f, x[f] + (f == 0 ? u : 0));
+          const AT df = z ? AT(0) : (p[u] - m[u]) * (rdx[u] * V(0.5));
+          if (k == ND - 1) acc[fE(ND)][u] -= df;
+          else acc[fB(ND, k < f ? k : k + 1)][u] -= df;
+        }
+      }
+      pin_acc();
+    };
+#pragma unroll
+    for (int f = 0; f < ND; f++) {
+      part1(f);
+      if (!ALL) {
+        __syncthreads();
+        const bool more = f + 1 < ND;
+        const SH* nq = ws + (long long)fB(ND, more ? f + 1 : 0) * N;
+        if (more) Q.load(G, nq, o);
+        part2(f);
+        if (more) {
+          Q.store(G, nq, QB(QM), o);
+          __syncthreads();
+        }
+      }
+    }
+    if (ALL) {
+      __syncthreads();
+#pragma unroll
+      for (int f = 0; f < ND; f++) part2(f);
+    }
+  }
+
+  if (!any) return;
+  // ------------------------------------------------------------ gravity
+  OT rho_c[XC], rhob_c[XC];
+  own(w, rho_c);
+  own(bg + (long long)bRHOB() * N, rhob_c);
+  if (T & SMAUG_T_GRAV) {
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+      if (G.g[d] == 0.0) continue;  // no gravity along d: both terms are zero
+      OT m1[XC];
+      own(w + (long long)fMOM(d) * N, m1);
+#pragma unroll
+      for (int u = 0; u < XC; u++) {
+        acc[fMOM(d)][u] += (AT)(G.g[d] * rho_c[u]);
+        acc[fE(ND)][u] += (AT)(rho_c[u] * (G.g[d] * m1[u]) / (rho_c[u] + rhob_c[u]));
+      }
+    }
+  }
+  // ------------------------------------------------------------ update, source, RK, ghosts
+  const double h = A.hfrac * A.dts[0];
+  const OT* __restrict__ base = (const OT*)A.base;
+  OT* __restrict__ wo = (OT*)A.wout;
+  OT outs[NP][XC];
+#pragma unroll
+  for (int f = 0; f < NP; f++) {
+    OT b1[XC];
+    own(base + (long long)f * N, b1);
+#pragma unroll
+    for (int u = 0; u < XC; u++) outs[f][u] = b1[u] + h * (OT)acc[f][u];
+  }
+#pragma unroll
+  for (int u = 0; u < XC; u++) {
+    if (!valid[u]) continue;
+    OT out[NP];
+#pragma unroll
+    for (int f = 0; f < NP; f++) out[f] = outs[f][u];
+    add_source<ND, OT>(G, A, T, x[0] + u, x[1], x[2], c + u, rho_c[u], rhob_c[u], h, out);
+#pragma unroll
+    for (int f = 0; f < NP; f++) outs[f][u] = out[f];
+  }
+  if (A.r1) {
+    if constexpr (XC == 2) {
+#pragma unroll
+      for (int f = 0; f < NP; f++) {
+        const long long o_f = (long long)f * N;
+        OT b0[XC], b1[XC], b2[XC], b3[XC];
+        own(base + o_f, b0);
+        own((const OT*)A.r1 + o_f, b1);
+        own((const OT*)A.r2 + o_f, b2);
+        own((const OT*)A.r3 + o_f, b3);
+#pragma unroll
+        for (int u = 0; u < XC; u++) outs[f][u] = outs[f][u] + (b1[u] + 2.0 * b2[u] + b3[u] - 4.0 * b0[u]) / 3;
+      }
+    } else {  // pointers per lane, stepped field by field, as in put_images
+      const OT *p0 = base + c, *p1 = (const OT*)A.r1 + c, *p2 = (const OT*)A.r2 + c, *p3 = (const OT*)A.r3 + c;
+#pragma unroll
+      for (int f = 0; f < NP; f++, p0 += N, p1 += N, p2 += N, p3 += N)
+        outs[f][0] = outs[f][0] + (*p1 + 2.0 * *p2 + *p3 - 4.0 * *p0) / 3;
+    }
+  }
+  // the cells themselves, then their ghost images
+  if (valid[XC - 1]) {
+#pragma unroll
+    for (int q = 0; q < NP; q++) stg<XC>(wo + (long long)q * N, c, outs[q]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < NP; q++) put(wo + (long long)q * N, c, outs[q][0]);
+  }
+  if (!EDGE) return;  // no cell of an inner tile has a ghost image
+#pragma unroll
+  for (int u = 0; u < XC; u++) {
+    if (!valid[u]) continue;
+    OT out[NP];
+#pragma unroll
+    for (int f = 0; f < NP; f++) out[f] = outs[f][u];
+    const int y[3] = {x[0] + u, x[1], x[2]};
+    put_images<ND, OT>(G, wo, y, out);
+  }
+}
+
+// Tiles of k_rhs_tiled.  FP64 and FP32: 8 x 4 x 8 in 3D (dim 0 contiguous and
+// 8 wide for coalesced rows; deep in z, the direction whose neighbour tiles
+// are least likely to still be in L2) and 16 x 16 in 2D.  Dual numbers are
+// twice as large in LDS, where one tile per CU fits: 8 x 8 x 8 cells give it
+// eight wavefronts to the four of the smaller tile (a tangent-linear step at
+// 96^3 4.29 -> 2.45 ms; FP32 pairs the same either way).
+template <int ND, typename SH>
+struct TileOf {
+  using T = TileT<3, 8, 4, 8, 1>;
+};
+template <typename SH>
+struct TileOf<2, SH> {
+  using T = TileT<2, 16, 16, 1, 1>;
+};
+template <>
+struct TileOf<3, Dual> {
+  using T = TileT<3, 8, 8, 8, 1>;
+};
+template <>
+struct TileOf<3, DualF> {
+  using T = TileT<3, 8, 8, 8, 1>;
+};
+// the tile of k_rhs_small
+using SmallTile = TileT<3, 8, 4, 8, 1>;
+// the tile of k_rhs_wide: two cells per thread
+using WideTile = TileT<3, 8, 8, 8, 2>;
+
+// origin of workgroup b's tile.  XCD-aware tile order: the hardware deals
+// consecutive workgroups to the 8 XCDs in turn, so workgroup b runs on XCD
+// b%8.  In 3D XCD x takes the slab of tile layers [x*gz/8, (x+1)*gz/8) and
+// walks it x fastest, then z, then y, so the z neighbour of a tile runs gx
+// tiles after it (its halo planes still in that XCD's L2) and the y
+// neighbour gx*gz/8 tiles after it (measured 1.7 % faster at 256^3 than x,
+// y, z order, whose z neighbour comes gx*gy tiles later); otherwise XCD x
+// takes the tiles [x*nb/8, (x+1)*nb/8) in x, y, z order.
+template <class TL>
+__device__ __forceinline__ void tile_origin(const Geo& G, int b, int* o) {
+  constexpr int ND = TL::ND, TX = TL::X, TY = TL::Y, TZ = TL::Z;
   const int gx = (G.n[0] - 4 + TX - 1) / TX, gy = (G.n[1] - 4 + TY - 1) / TY;
   const int gz = ND == 3 ? (G.n[2] - 4 + TZ - 1) / TZ : 1;
   const int nb = gx * gy * gz;
-  const int b = blockIdx.x;
   int t = b;
   if ((nb & 7) == 0) {
     const int xcd = b & 7, tl = b >> 3;
@@ -907,25 +1294,135 @@ __global__ __launch_bounds__(256, sizeof(SH) == 4 ? 5 : (std::is_same<SH, double
       t = xcd * (nb >> 3) + tl;
     }
   }
-  const int tbx = t % gx, tby = (t / gx) % gy, tbz = t / (gx * gy);
-  const int o[3] = {2 + tbx * TX, 2 + tby * TY, ND == 3 ? 2 + tbz * TZ : 0};
-  // inner tile: every cell in [5, n-6] along every direction (the test is
-  // uniform per workgroup; the first and last tile layer along an axis are
-  // edge tiles)
-  bool edge = o[0] < 5 || o[0] + TX - 1 > G.n[0] - 6 || o[1] < 5 || o[1] + TY - 1 > G.n[1] - 6;
-  if (ND == 3) edge = edge || o[2] < 5 || o[2] + TZ - 1 > G.n[2] - 6;
-  if (edge)
-    rhs_tile<ND, SH, true>(G, A, sm, o);
-  else
-    rhs_tile<ND, SH, false>(G, A, sm, o);
+  o[0] = 2 + t % gx * TX;
+  o[1] = 2 + (t / gx) % gy * TY;
+  o[2] = ND == 3 ? 2 + t / (gx * gy) * TZ : 0;
 }
+
+// inner tile: every cell in [5, n-6] along every direction (the test is
+// uniform per workgroup; the first and last tile layer along an axis are
+// edge tiles)
+template <class TL>
+__device__ __forceinline__ bool edge_tile(const Geo& G, const int* o) {
+  bool edge = o[0] < 5 || o[0] + TL::X - 1 > G.n[0] - 6 || o[1] < 5 || o[1] + TL::Y - 1 > G.n[1] - 6;
+  if (TL::ND == 3) edge = edge || o[2] < 5 || o[2] + TL::Z - 1 > G.n[2] - 6;
+  return edge;
+}
+
+template <class TL>
+static int tiles_of(const Geo& G) {
+  int nb = ((G.n[0] - 4 + TL::X - 1) / TL::X) * ((G.n[1] - 4 + TL::Y - 1) / TL::Y);
+  if (TL::ND == 3) nb *= (G.n[2] - 4 + TL::Z - 1) / TL::Z;
+  return nb;
+}
+
+// wavefronts per SIMD the registers must allow
+template <int ND, typename SH>
+constexpr int min_waves() {
+  return ND == 2 ? 2 : (sizeof(SH) == 4 ? 5 : (std::is_same<SH, double>::value ? 4 : 2));
+}
+
+// One cell per thread, on a tensor-product grid.  2D tiles keep every box in
+// LDS (36 KB in FP64), 3D ones the boxes of a phase.
+template <int ND, typename SH>
+__global__ __launch_bounds__((TileOf<ND, SH>::T::NT), (min_waves<ND, SH>())) void k_rhs_tiled(Geo G, RhsArgs A) {
+  using TL = typename TileOf<ND, SH>::T;
+  constexpr bool ALL = ND == 2;
+  __shared__ __align__(16) SH sm[ALL ? Lay<TL>::SMEM_ALL : Lay<TL>::SMEM];
+  if (A.zero_next && blockIdx.x == 0 && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  int o[3];
+  tile_origin<TL>(G, blockIdx.x, o);
+  if (edge_tile<TL>(G, o))
+    rhs_tile<TL, SH, true, true, ALL>(G, A, sm, o);
+  else
+    rhs_tile<TL, SH, false, true, ALL>(G, A, sm, o);
+}
+
+// the same on any other grid (a kernel of its own: with both in one the
+// tensor-product grids ran 2 to 6 % slower)
+template <int ND, typename SH>
+__global__ __launch_bounds__((TileOf<ND, SH>::T::NT), (min_waves<ND, SH>())) void k_rhs_general(Geo G, RhsArgs A) {
+  using TL = typename TileOf<ND, SH>::T;
+  __shared__ __align__(16) SH sm[Lay<TL>::SMEM];
+  if (A.zero_next && blockIdx.x == 0 && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  int o[3];
+  tile_origin<TL>(G, blockIdx.x, o);
+  if (edge_tile<TL>(G, o))
+    rhs_tile<TL, SH, true, false, false>(G, A, sm, o);
+  else
+    rhs_tile<TL, SH, false, false, false>(G, A, sm, o);
+}
+
+// 3D tensor-product grids of few tiles: every box of a tile in LDS at once
+// (158 KB in FP64).  A tile that has a CU to itself waits for memory and
+// barriers most of its time: 48 us for the phases one after the other, 33 us
+// this way (FP64, 16x12x12; 0.205 -> 0.144 ms per step).
+template <typename SH>
+__global__ __launch_bounds__(SmallTile::NT, 1) void k_rhs_small(Geo G, RhsArgs A) {
+  using TL = SmallTile;
+  __shared__ __align__(16) SH sm[Lay<TL>::SMEM_ALL];
+  if (A.zero_next && blockIdx.x == 0 && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  int o[3];
+  tile_origin<TL>(G, blockIdx.x, o);
+  if (edge_tile<TL>(G, o))
+    rhs_tile<TL, SH, true, true, true>(G, A, sm, o);
+  else
+    rhs_tile<TL, SH, false, true, true>(G, A, sm, o);
+}
+
+// FP64 on large 3D tensor-product grids: two cells per thread, 8 x 8 x 8
+// tiles, three workgroups per CU (168 VGPRs, 53.5 KB of LDS).
+__global__ __launch_bounds__(WideTile::NT, 3) void k_rhs_wide(Geo G, RhsArgs A) {
+  using TL = WideTile;
+  __shared__ __align__(16) double sm[Lay<TL>::SMEM];
+  if (A.zero_next && blockIdx.x == 0 && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  int o[3];
+  tile_origin<TL>(G, blockIdx.x, o);
+  if (edge_tile<TL>(G, o))
+    rhs_tile<TL, double, true, true, false>(G, A, sm, o);
+  else
+    rhs_tile<TL, double, false, true, false>(G, A, sm, o);
+}
+
+// (the tests compile the dispatch with other limits, to send every grid
+// through each kernel)
+#ifndef SMAUG_CUS
+#define SMAUG_CUS 256
+#endif
+#ifndef SMAUG_WIDE_TILES
+#define SMAUG_WIDE_TILES 12000
+#endif
+constexpr int kLds = 160 * 1024;  // LDS of a CU
 
 template <int ND, typename SH>
 static void launch_tiled_t(const Geo& G, hipStream_t st, const RhsArgs& A) {
-  using L = Lay<ND>;
-  int nb = ((G.n[0] - 4 + L::TX - 1) / L::TX) * ((G.n[1] - 4 + L::TY - 1) / L::TY);
-  if (ND == 3) nb *= (G.n[2] - 4 + L::TZ - 1) / L::TZ;
-  hipLaunchKernelGGL((k_rhs_tiled<ND, SH>), dim3(nb), dim3(256), 0, st, G, A);
+  using TL = typename TileOf<ND, SH>::T;
+  constexpr int fit = kLds / (int)(sizeof(SH) * Lay<SmallTile>::SMEM_ALL);  // k_rhs_small tiles per CU
+  const int nb = tiles_of<TL>(G);
+  if (!A.dx1) {
+    hipLaunchKernelGGL((k_rhs_general<ND, SH>), dim3(nb), dim3(TL::NT), 0, st, G, A);
+    return;
+  }
+  if constexpr (ND == 3 && fit > 0) {
+    // as long as the whole grid is resident at once: FP64 40^3 (250 tiles)
+    // 0.041 against 0.054 ms, 48^3 (432) 0.064 against 0.059; FP32, two per
+    // CU, 48^3 0.038 against 0.053, 56^3 (686) 0.073 against 0.070
+    if (tiles_of<SmallTile>(G) <= SMAUG_CUS * fit) {
+      hipLaunchKernelGGL((k_rhs_small<SH>), dim3(tiles_of<SmallTile>(G)), dim3(SmallTile::NT), 0, st, G, A);
+      return;
+    }
+  }
+  if constexpr (std::is_same<SH, double>::value && ND == 3) {
+    // two cells per thread pay once the grid is many rounds of tiles: 128^3
+    // (4096 wide tiles) 0.513 ms either way, 160^3 (8000) 0.996 against 0.995,
+    // 192^3 (13824) 1.541 against 1.596, 256^3 3.51 against 3.73; at 96^3
+    // 0.246 against 0.231
+    if (tiles_of<WideTile>(G) >= SMAUG_WIDE_TILES) {
+      hipLaunchKernelGGL(k_rhs_wide, dim3(tiles_of<WideTile>(G)), dim3(WideTile::NT), 0, st, G, A);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_rhs_tiled<ND, SH>), dim3(nb), dim3(TL::NT), 0, st, G, A);
 }
 
 // the tangent-linear stage: every state array of A (win, base, r1..r3,
