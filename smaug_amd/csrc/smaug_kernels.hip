@@ -23,6 +23,19 @@ namespace smaug {
 
 __device__ inline double bits2d(unsigned long long b) { return __longlong_as_double((long long)b); }
 
+// *p = max(*p, t) for t >= 0 by its bits.  The atomics of all blocks meet on
+// three addresses and pass one at a time (some 10 ns each), which took a 3D
+// pass over 10^5 to 10^7 cells longer than its traffic: 84 us at 96^3, 80 us
+// at 101x75x61.  With many blocks each reads the value first and leaves out an
+// atomic that cannot raise it (a stale value is only smaller), and there are
+// at most 1024 of them: 40 and 29 us.  With few the read is one more trip:
+// 13.3 against 12.8 us at 32^3 (183 blocks); 14.2 against 18.8 us at 256x512
+// (529 blocks).
+__device__ inline void raise_max(unsigned long long* p, double t) {
+  const unsigned long long v = (unsigned long long)__double_as_longlong(t);
+  if (t > 0.0 && (gridDim.x <= 256 || v > *(volatile unsigned long long*)p)) atomicMax(p, v);
+}
+
 // ---------------------------------------------------------------------------
 // k_prim: pointwise derived fields + wave-speed maxima
 //   v_d  = m_d/(rho+rhob)                         src/dervfields.cu:79-98
@@ -127,7 +140,7 @@ __global__ __launch_bounds__(256) void k_prim(Geo G, const double* __restrict__ 
     for (int d = 0; d < ND; d++) {
       double t = red[0][d];
       for (int q = 1; q < 4; q++) t = red[q][d] > t ? red[q][d] : t;
-      if (t > 0.0) atomicMax(&cmax_bits[d], (unsigned long long)__double_as_longlong(t));
+      raise_max(&cmax_bits[d], t);
     }
   }
 }
@@ -219,7 +232,7 @@ __global__ __launch_bounds__(256) void k_prim_tl(Geo G, const Dual* __restrict__
     for (int d = 0; d < ND; d++) {
       double t = red[0][d];
       for (int q = 1; q < 4; q++) t = red[q][d] > t ? red[q][d] : t;
-      if (t > 0.0) atomicMax(&cmax_bits[d], (unsigned long long)__double_as_longlong(t));
+      raise_max(&cmax_bits[d], t);
     }
   }
 }
@@ -309,9 +322,10 @@ __global__ __launch_bounds__(256) void k_fill(Geo G, double* __restrict__ w) {
 
 void launch_prim(const Geo& G, hipStream_t st, const double* w, const double* bg, void* prim, float* shadow,
                  unsigned long long* cmax, int* flag) {
-  // grid-stride: at most 2048 blocks so the per-block atomics stay few
+  // grid-stride: at most 1024 blocks so the per-block atomics stay few (see
+  // raise_max)
   long long nb = (G.N + 255) / 256;
-  if (nb > 2048) nb = 2048;
+  if (nb > 1024) nb = 1024;
   if (G.mixed) {
     if (G.nd == 3)
       hipLaunchKernelGGL((k_prim<3, float>), dim3((unsigned)nb), dim3(256), 0, st, G, w, bg, (float*)prim, shadow,
@@ -332,7 +346,7 @@ void launch_prim(const Geo& G, hipStream_t st, const double* w, const double* bg
 void launch_prim_tl(const Geo& G, hipStream_t st, const Dual* w, const Dual* bg, void* prim, void* shadow,
                     unsigned long long* cmax, int* flag) {
   long long nb = (G.N + 255) / 256;
-  if (nb > 2048) nb = 2048;
+  if (nb > 1024) nb = 1024;
   const dim3 g((unsigned)nb), b(256);
   if (G.mixed) {
     if (G.nd == 3)
