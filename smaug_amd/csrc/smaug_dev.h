@@ -215,6 +215,20 @@ __host__ __device__ __forceinline__ long long halo_r_src(const Geo& G, const int
   return h;
 }
 
+// CFL step (src/iosmaug.c:541-616, quirk Q4): the last direction's maximum
+// cm over every dir's dx; the step starts from DT (dt=DT, p->dt=DT, :549-550)
+// and takes the CFL step when it lies in (1e-12, DT) (:568-569)
+__host__ __device__ __forceinline__ double cfl_dt(double cm, int nd, double dx0, double dx1, double dx2, double courant,
+                                                  double dtcap) {
+  double courantmax = 1.0e-12;
+  for (int d = 0; d < nd; d++) {
+    const double t = cm / (d == 0 ? dx0 : (d == 1 ? dx1 : dx2));
+    if (t > courantmax) courantmax = t;
+  }
+  const double dtt = courant / courantmax;
+  return dtt > 1.0e-12 && dtt < dtcap ? dtt : dtcap;
+}
+
 struct RhsArgs {
   const double* win;    // stage input, evolved fields (FP64, own-cell values)
   const void* wsh;      // stage input as the stencils read it: win itself
@@ -233,7 +247,11 @@ struct RhsArgs {
   double* wout;
   const unsigned long long* cmax_bits;  // this stage's maxima
   unsigned long long* zero_next;        // maxima slot of the next stage
-  const double* dts;                    // device dt
+  double* dts;                          // device (dt, t)
+  int dt_rule;                          // 0: dt is dts[0]; the step's first stage also
+                                        // advances the clock: 1 by dts[0], 2 by the
+                                        // CFL step of this stage's maxima, kept in dts[0]
+  double courant, dtcap;                // of the CFL rule
   double hfrac;                         // stage step = hfrac*dt
   double tdep;                          // driver time factor sin(2 pi qt/P)
   double damp;                          // tangent of the driver amplitude drv[0]

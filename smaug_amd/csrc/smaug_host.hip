@@ -471,6 +471,9 @@ static RhsArgs rhs_args(smaug_t* s, const double* win, const double* base, doubl
   A.cmax_bits = s->cmax + 4 * slot;
   A.zero_next = s->cmax + 4 * (slot ^ 1);
   A.dts = s->dts;
+  A.dt_rule = 0;
+  A.courant = s->p.courant;
+  A.dtcap = s->p.dt;
   A.hfrac = hfrac;
   A.tdep = tdep;
   A.damp = 0.0;
@@ -479,14 +482,16 @@ static RhsArgs rhs_args(smaug_t* s, const double* win, const double* base, doubl
   return A;
 }
 
+// rule by which the first stage of a step sets dt and the clock (RhsArgs)
+static int dt_rule(const smaug_t* s) { return s->p.moddton == 1 ? 2 : 1; }
+
 // one stage: prim of win into the current maxima slot, then the rhs
 static void run_stage(smaug_t* s, const double* win, const double* base, double* wout, double hfrac, double tdep,
                       bool first, const double* r1, const double* r2, const double* r3) {
   const int slot = s->cslot;
   launch_prim(s->G, s->stream, win, s->bg, s->prim, s->shadow, s->cmax + 4 * slot, s->flag);
-  if (first)
-    launch_dt(s->stream, s->cmax + 4 * slot, s->nd, s->p.dx, s->p.courant, s->p.dt, s->p.moddton, s->dts);
   RhsArgs A = rhs_args(s, win, base, wout, hfrac, tdep, slot);
+  if (first) A.dt_rule = dt_rule(s);
   A.r1 = r1;
   A.r2 = r2;
   A.r3 = r3;
@@ -1011,8 +1016,6 @@ static void tl_stage(smaug_t* s, const Geo& Gt, Dual* win, const Dual* base, Dua
   hipStream_t st = s->stream;
   const int slot = s->tlslot;
   launch_prim_tl(Gt, st, win, s->tlbg, s->tlprim, s->tlshadow, s->tlcmax + 4 * slot, s->flag);
-  if (first)
-    launch_dt(st, s->tlcmax + 4 * slot, s->nd, s->p.dx, s->p.courant, s->p.dt, s->p.moddton, s->tldts);
   RhsArgs A;
   A.win = (const double*)win;
   A.wsh = Gt.mixed ? (const void*)s->tlshadow : (const void*)win;
@@ -1031,6 +1034,9 @@ static void tl_stage(smaug_t* s, const Geo& Gt, Dual* win, const Dual* base, Dua
   A.cmax_bits = s->tlcmax + 4 * slot;
   A.zero_next = s->tlcmax + 4 * (slot ^ 1);
   A.dts = s->tldts;
+  A.dt_rule = first ? dt_rule(s) : 0;
+  A.courant = s->p.courant;
+  A.dtcap = s->p.dt;
   A.hfrac = hfrac;
   A.tdep = tdep;
   A.damp = s->tldamp;
@@ -1129,9 +1135,8 @@ extern "C" int smaug_time_kernels(smaug_t* s, int nsteps, double* ms_prim, doubl
       HIPCHK(hipEventRecord(ev[4 * st + 0], s->stream));
       launch_prim(s->G, s->stream, win, s->bg, s->prim, s->shadow, s->cmax + 4 * slot, s->flag);
       HIPCHK(hipEventRecord(ev[4 * st + 1], s->stream));
-      if (st == 0)
-        launch_dt(s->stream, s->cmax + 4 * slot, s->nd, s->p.dx, s->p.courant, s->p.dt, s->p.moddton, s->dts);
       RhsArgs A = rhs_args(s, win, base, wout, hf, tdep, slot);
+      if (st == 0) A.dt_rule = dt_rule(s);
       A.r1 = r1;
       A.r2 = r2;
       A.r3 = r3;

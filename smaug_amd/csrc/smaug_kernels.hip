@@ -11,8 +11,8 @@
 //           hyperdiffusion coefficients and sources, the stage update, the
 //           user source on the updated state, the RK combination and the
 //           ghost fill.
-// The CFL time step is chosen on the device by k_dt so a step needs no
-// host round trip.
+// The CFL time step is chosen on the device, by the first stage's k_rhs, so a
+// step needs no host round trip.
 #include <math.h>
 
 #include "../../include/smaug_hip.h"
@@ -259,27 +259,13 @@ __global__ void k_clear_flag(int* flag) {
   if (threadIdx.x == 0) *flag = 0;
 }
 
-// CFL step (src/iosmaug.c:541-616, quirk Q4): the last direction's maximum
-// over every dir's dx.  With moddton=1 each step starts from DT (dt=DT,
-// p->dt=DT, :549-550) and takes the CFL step when it lies in (1e-12, DT)
-// (:568-569); otherwise the step keeps its value.  dts[0] = dt, dts[1] =
-// accumulated time.
+// The time step by itself (smaug_cfl_noalloc; the time loop's first stage
+// does this in k_rhs): with moddton=1 the CFL step, otherwise the step keeps
+// its value.  dts[0] = dt, dts[1] = accumulated time.
 __global__ void k_dt(const unsigned long long* cmax_bits, int nd, double dx0, double dx1, double dx2,
                      double courant, double dtcap, int moddton, double* dts) {
   if (threadIdx.x != 0) return;
-  double dt = dts[0];
-  if (moddton == 1) {
-    const double cm = bits2d(cmax_bits[nd - 1]);
-    const double dxs[3] = {dx0, dx1, dx2};
-    double courantmax = 1.0e-12;
-    for (int d = 0; d < nd; d++) {
-      double t = cm / dxs[d];
-      if (t > courantmax) courantmax = t;
-    }
-    dt = dtcap;
-    const double dtt = courant / courantmax;
-    if (dtt > 1.0e-12 && dtt < dtcap) dt = dtt;
-  }
+  const double dt = moddton == 1 ? cfl_dt(bits2d(cmax_bits[nd - 1]), nd, dx0, dx1, dx2, courant, dtcap) : dts[0];
   dts[0] = dt;
   dts[1] = dts[1] + dt;
 }

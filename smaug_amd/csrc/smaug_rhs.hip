@@ -313,6 +313,28 @@ struct Win {
   }
 };
 
+// The stage's dt.  The CFL rule is evaluated by every workgroup of the step's
+// first stage, from the maxima that stage uses, rather than by a kernel of its
+// own before it: 8 launches per RK4 step for 9, 2 per single-stage step for 3.
+__device__ __forceinline__ double stage_dt(const Geo& G, const RhsArgs& A) {
+  if (A.dt_rule != 2) return A.dts[0];
+  return cfl_dt(__longlong_as_double((long long)A.cmax_bits[G.nd - 1]), G.nd, G.pdx[0], G.pdx[1], G.pdx[2], A.courant,
+                A.dtcap);
+}
+
+// once per launch: the next stage's maxima back to zero, and in the step's
+// first stage the clock (dts[0] is written under rule 2 only, where no
+// workgroup reads it)
+__device__ __forceinline__ void stage_head(const Geo& G, const RhsArgs& A) {
+  if (blockIdx.x != 0) return;
+  if (A.zero_next && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  if (A.dt_rule != 0 && threadIdx.x == 0) {
+    const double dt = stage_dt(G, A);
+    if (A.dt_rule == 2) A.dts[0] = dt;
+    A.dts[1] = A.dts[1] + dt;
+  }
+}
+
 // The user source and the divB terms of one interior cell (x0, x1, x2) with
 // index c, on its updated values out.
 template <int ND, typename OT>
@@ -1180,7 +1202,7 @@ __device__ __forceinline__ void rhs_tile(const Geo& G, const RhsArgs& A, SH* __r
     }
   }
   // ------------------------------------------------------------ update, source, RK, ghosts
-  const double h = A.hfrac * A.dts[0];
+  const double h = A.hfrac * stage_dt(G, A);
   const OT* __restrict__ base = (const OT*)A.base;
   OT* __restrict__ wo = (OT*)A.wout;
   OT outs[NP][XC];
@@ -1329,7 +1351,7 @@ __global__ __launch_bounds__((TileOf<ND, SH>::T::NT), (min_waves<ND, SH>())) voi
   using TL = typename TileOf<ND, SH>::T;
   constexpr bool ALL = ND == 2;
   __shared__ __align__(16) SH sm[ALL ? Lay<TL>::SMEM_ALL : Lay<TL>::SMEM];
-  if (A.zero_next && blockIdx.x == 0 && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  stage_head(G, A);
   int o[3];
   tile_origin<TL>(G, blockIdx.x, o);
   if (edge_tile<TL>(G, o))
@@ -1344,7 +1366,7 @@ template <int ND, typename SH>
 __global__ __launch_bounds__((TileOf<ND, SH>::T::NT), (min_waves<ND, SH>())) void k_rhs_general(Geo G, RhsArgs A) {
   using TL = typename TileOf<ND, SH>::T;
   __shared__ __align__(16) SH sm[Lay<TL>::SMEM];
-  if (A.zero_next && blockIdx.x == 0 && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  stage_head(G, A);
   int o[3];
   tile_origin<TL>(G, blockIdx.x, o);
   if (edge_tile<TL>(G, o))
@@ -1361,7 +1383,7 @@ template <typename SH>
 __global__ __launch_bounds__(SmallTile::NT, 1) void k_rhs_small(Geo G, RhsArgs A) {
   using TL = SmallTile;
   __shared__ __align__(16) SH sm[Lay<TL>::SMEM_ALL];
-  if (A.zero_next && blockIdx.x == 0 && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  stage_head(G, A);
   int o[3];
   tile_origin<TL>(G, blockIdx.x, o);
   if (edge_tile<TL>(G, o))
@@ -1375,7 +1397,7 @@ __global__ __launch_bounds__(SmallTile::NT, 1) void k_rhs_small(Geo G, RhsArgs A
 __global__ __launch_bounds__(WideTile::NT, 3) void k_rhs_wide(Geo G, RhsArgs A) {
   using TL = WideTile;
   __shared__ __align__(16) double sm[Lay<TL>::SMEM];
-  if (A.zero_next && blockIdx.x == 0 && threadIdx.x < 3) A.zero_next[threadIdx.x] = 0ull;
+  stage_head(G, A);
   int o[3];
   tile_origin<TL>(G, blockIdx.x, o);
   if (edge_tile<TL>(G, o))
