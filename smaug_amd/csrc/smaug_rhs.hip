@@ -31,7 +31,7 @@
 //    by phase (pin) and loads of the own cell repeated rather than kept, which
 //    took the FP64 kernel from 150 to 109 VGPRs, and its LDS from 52 to 34 KB:
 //    four workgroups per CU instead of three (FP64, k_rhs at 128^3: 0.676 ->
-//    0.513 ms; FP32 0.470 -> 0.403);
+//    0.510 ms; FP32 0.470 -> 0.411);
 //  * the code of a tile at the grid's edge (masks, halo substitutions, ghost
 //    images) streamed 211 KB of instructions through caches of 64 KB per two
 //    CUs; loops in place of unrolled bodies made it 50 KB (one tile by itself:
@@ -40,8 +40,8 @@
 //    in LDS at once (ALL: 6 barriers for 20, 48 -> 33 us per tile);
 //  * on large FP64 grids the traffic of the boxes counts: a tile of twice the
 //    cells re-reads a third less halo (k_rhs at 256^3: 4.60 ms before, 3.73
-//    with the small tile, 3.51 with the wide one; 14.9 GB fetched from beyond
-//    L2 at 4.2 TB/s, of 5.0 TB/s that a streaming pass reaches).
+//    with the small tile, 3.49 with the wide one; 15.1 GB fetched from beyond L2
+//    and 1.3 GB written, 4.7 TB/s of the 5.0 that a streaming pass reaches).
 #include <math.h>
 
 #include <type_traits>
