@@ -41,7 +41,7 @@
 //  * on large FP64 grids the traffic of the boxes counts: a tile of twice the
 //    cells re-reads a third less halo (k_rhs at 256^3: 4.60 ms before, 3.73
 //    with the small tile, 3.49 with the wide one; 15.1 GB fetched from beyond L2
-//    and 1.3 GB written, 4.7 TB/s of the 5.0 that a streaming pass reaches).
+//    and 1.7 GB written, 4.8 TB/s of the 5.0 that a streaming pass reaches).
 #include <math.h>
 
 #include <type_traits>
