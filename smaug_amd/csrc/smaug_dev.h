@@ -157,12 +157,10 @@ __host__ __device__ __forceinline__ Img2 bc_images2(int type, int y, int n, int 
     if (y == n - 3) return Img2{1, n - 2, 0};
     return Img2{0, 0, 0};
   }
-  // contcd4; symm/asymm in 3D
-  if (y == 4) return Img2{1, 0, 0};
-  if (y == 3) return Img2{1, 1, 0};
-  if (y == n - 5) return Img2{1, n - 1, 0};
-  if (y == n - 4) return Img2{1, n - 2, 0};
-  return Img2{0, 0, 0};
+  // contcd4; symm/asymm in 3D.  The coordinates 3, 4 and n-5, n-4 overlap for
+  // n = 8 and 9: one of them feeds a ghost on either side
+  const int lo = y == 4 ? 0 : (y == 3 ? 1 : -1), hi = y == n - 5 ? n - 1 : (y == n - 4 ? n - 2 : -1);
+  return Img2{(lo >= 0) + (hi >= 0), lo >= 0 ? lo : hi, hi};
 }
 
 // zeroing of grad3dn at interior cells: first/last two interior layers

@@ -94,6 +94,30 @@ def test_3d_boundaries_terms_and_other_grids(libs, route):
     assert errors(libs[route], "start", "strat", (17, 12, 10), 1, 1, 1, 4, 0xFF) <= 1e-5
 
 
+# 4 and 5 interior cells along an axis (the smallest the engine takes): a cell
+# there feeds a ghost on either side, two in all.  (The stratified atmosphere
+# on so few cells along dim 0 is stable with the single-stage scheme only: RK4
+# takes the oracle to negative densities within two steps.)
+SMALLEST = [(4, 4, 4), (5, 5, 5), (12, 4, 5), (5, 12, 4), (4, 5, 12)]
+
+
+@pytest.mark.parametrize("route", list(ROUTES))
+def test_smallest_3d_grids(libs, route):
+    for ni in SMALLEST:
+        for bc in (3, 4, 5, 6, 7):  # cont, contcd4, fixed, symm, asymm
+            assert errors(libs[route], "end", "strat", ni, 0, 0, 0, bc, 0xFF) <= 1e-12, (ni, bc)
+        assert errors(libs[route], "start", "strat", ni, 0, 1, 0, 4, 0xFF) <= 1e-5, ni
+    assert errors(libs[route], "start", "strat", (12, 4, 5), 1, 0, 0, 4, 0xFF) <= 1e-12
+
+
+def test_smallest_2d_grids(libs):
+    for ni in ((4, 4), (5, 4), (4, 17), (16, 5)):
+        for bc in (3, 4, 5, 6, 7):
+            assert errors(libs["tiled"], "end", "strat", ni, int(ni[0] > 8), 0, 0, bc, 0xFF) <= 1e-12, (ni, bc)
+    for n in (4, 5):
+        assert errors(libs["tiled"], "end", "ot", (n, n), 1, 0, 0, 0, 0xFF) <= 1e-12, n
+
+
 def test_2d_grids(libs):
     for ni in ((12, 6), (16, 16), (17, 33), (31, 48)):
         assert errors(libs["tiled"], "end", "strat", ni, 1, 0, 0, 4, 0xFF) <= 1e-12, ni
@@ -104,11 +128,11 @@ def test_2d_grids(libs):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("ni,mixed", [((40, 40, 40), 0), ((41, 40, 40), 0), ((40, 40, 40), 1), ((64, 64, 33), 1),
+@pytest.mark.parametrize("ni,mixed", [((4, 4, 4), 0), ((5, 12, 4), 0), ((12, 4, 5), 1), ((40, 40, 40), 0), ((41, 40, 40), 0), ((40, 40, 40), 1), ((64, 64, 33), 1),
                                       ((184, 184, 184), 0)])
 def test_routes_on_the_gpu(ni, mixed):
-    """Both sides of the limits in FP64 and FP32, and the wide kernel on a
-    grid whose rows are not aligned."""
+    """The smallest grids, both sides of the limits in FP64 and FP32, and the
+    wide kernel on a grid whose rows are not aligned."""
     from oracle.pyoracle import Oracle
     from smaug_amd.engine import Engine
     from tests.cases import compare, strat_case
