@@ -1235,6 +1235,15 @@ __device__ __forceinline__ void rhs_tile(const Geo& G, const RhsArgs& A, SH* __r
         own((const OT*)A.r3 + o_f, b3);
 #pragma unroll
         for (int u = 0; u < XC; u++) outs[f][u] = outs[f][u] + (b1[u] + 2.0 * b2[u] + b3[u] - 4.0 * b0[u]) / 3;
+        // in two halves: with the loads of every field in flight at once the
+        // registers of three workgroups per CU do not hold them (16 went to
+        // scratch memory, which the runtime has to set up for a first launch)
+        if (f == NP / 2 - 1) {
+#pragma unroll
+          for (int g = 0; g <= f; g++)
+#pragma unroll
+            for (int u = 0; u < XC; u++) pin(outs[g][u]);
+        }
       }
     } else {  // pointers per lane, stepped field by field, as in put_images
       const OT *p0 = base + c, *p1 = (const OT*)A.r1 + c, *p2 = (const OT*)A.r2 + c, *p3 = (const OT*)A.r3 + c;

@@ -1,11 +1,13 @@
-"""Register budget of the stage kernel (CPU: compiles smaug_rhs.hip for
-gfx950 and reads the compiler's resource report).  The FP64 k_rhs is tuned
-for three wavefronts per SIMD with no scratch: 169 VGPRs already halve the
-number of resident tiles (measured: 6.6 -> 8.6 ms per launch at 256^3), so a
-change that crosses 168 must show up here rather than in the benchmark.  The
-FP32 (mixed-precision) k_rhs runs five wavefronts per SIMD with at most a
-small spill (measured: 4.0 ms against 4.3 ms at four wavefronts without a
-spill and 4.6 ms at six with a 72-byte spill)."""
+"""Register, LDS and scratch budget of the kernels (CPU: compiles the sources
+for gfx950 and reads the compiler's resource report).
+
+The stage kernels are tuned for a number of workgroups resident per CU, which
+their registers and their LDS have to allow together: FP64 k_rhs_tiled four in
+3D (0.676 -> 0.510 ms per launch at 128^3 when it went from three), FP32 five,
+k_rhs_wide three, k_rhs_small two in FP32 (its dispatch counts on them).  A
+change that crosses one of those lines must show up here rather than in the
+benchmark.  None of the 20 uses scratch memory: the runtime sets that up at a
+kernel's first launch on a stream."""
 from __future__ import annotations
 
 import os
@@ -35,38 +37,55 @@ def resources(src_name, tmp_path):
             name = m.group(1)
             report[name] = {}
             continue
-        m = re.search(r"remark:\s+(VGPRs|AGPRs|ScratchSize \[bytes/lane\]|Occupancy \[waves/SIMD\]): (\d+)", line)
+        m = re.search(r"remark:\s+(VGPRs|AGPRs|ScratchSize \[bytes/lane\]|Occupancy \[waves/SIMD\]|LDS Size \[bytes/block\]): (\d+)", line)
         if m and name:
             report[name][m.group(1).split()[0]] = int(m.group(2))
     return report
+
+
+# kernel (mangled name part): threads, workgroups a CU has to hold
+LDS_PER_CU = 160 * 1024
+STAGE_KERNELS = {
+    "k_rhs_tiledILi3EdE": (256, 4),
+    "k_rhs_tiledILi3EfE": (256, 5),
+    "k_rhs_tiledILi3ENS_4DualEE": (512, 1),
+    "k_rhs_tiledILi3ENS_5DualFEE": (512, 2),
+    "k_rhs_tiledILi2EdE": (256, 4),
+    "k_rhs_tiledILi2EfE": (256, 4),
+    "k_rhs_tiledILi2ENS_4DualEE": (256, 2),
+    "k_rhs_tiledILi2ENS_5DualFEE": (256, 4),
+    "k_rhs_generalILi3EdE": (256, 4),
+    "k_rhs_generalILi3EfE": (256, 5),
+    "k_rhs_generalILi3ENS_4DualEE": (512, 1),
+    "k_rhs_generalILi3ENS_5DualFEE": (512, 2),
+    "k_rhs_generalILi2EdE": (256, 4),
+    "k_rhs_generalILi2EfE": (256, 4),
+    "k_rhs_generalILi2ENS_4DualEE": (256, 2),
+    "k_rhs_generalILi2ENS_5DualFEE": (256, 4),
+    "k_rhs_smallIdE": (256, 1),
+    "k_rhs_smallIfE": (256, 2),
+    "k_rhs_smallINS_5DualFEE": (256, 1),
+    "k_rhs_wideE": (256, 3),
+}
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
 def test_k_rhs_occupancy_and_scratch(tmp_path):
     from smaug_amd.build import ARCH
 
-    report = resources("smaug_rhs.hip", tmp_path)
-    k64 = {k: v for k, v in report.items() if "k_rhs_tiledILi3EdE" in k}
-    k32 = {k: v for k, v in report.items() if "k_rhs_tiledILi3EfE" in k}
-    assert len(k64) == 1 and len(k32) == 1, report
-    for k, v in k64.items():
-        assert v["Occupancy"] >= 3, (k, v)
-        assert v["ScratchSize"] == 0, (k, v)
-    for k, v in k32.items():
-        assert v["Occupancy"] >= 5, (k, v)
-        assert v["ScratchSize"] <= 16, (k, v)
-    # the tangent-linear (Dual) instantiations: no scratch; the 3D one's
-    # 105 KB of LDS allow one workgroup per CU, so its registers may run into
-    # the accumulation file (256 + 10 at gfx950); the mixed-precision ones
-    # (DualF) keep two wavefronts per SIMD or more
-    kd = {k: v for k, v in report.items() if "k_rhs_tiled" in k and "4DualE" in k}
-    kf = {k: v for k, v in report.items() if "k_rhs_tiled" in k and "5DualFE" in k}
-    assert len(kd) == 2 and len(kf) == 2, report
-    for k, v in kd.items():
-        assert v["VGPRs"] + v.get("AGPRs", 0) <= 512 and v["ScratchSize"] == 0, (k, v)
-    for k, v in kf.items():
-        assert v["Occupancy"] >= 2 and v.get("AGPRs", 0) == 0 and v["ScratchSize"] == 0, (k, v)
     assert ARCH == "gfx950"
+    report = resources("smaug_rhs.hip", tmp_path)
+    found = {}
+    for part in STAGE_KERNELS:
+        names = [k for k in report if part in k]
+        assert len(names) == 1, (part, names)
+        found[names[0]] = part
+    assert set(found) == set(report), set(report) - set(found)  # every stage kernel is listed
+    for name, part in found.items():
+        v, (threads, groups) = report[name], STAGE_KERNELS[part]
+        assert v["ScratchSize"] == 0, (part, v)
+        assert v["Occupancy"] * 4 * 64 >= groups * threads, (part, v)
+        assert v["LDS"] * groups <= LDS_PER_CU, (part, v)
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
