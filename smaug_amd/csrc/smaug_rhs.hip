@@ -1437,8 +1437,14 @@ static void launch_tiled_t(const Geo& G, hipStream_t st, const RhsArgs& A) {
   if constexpr (ND == 3 && fit > 0) {
     // as long as the whole grid is resident at once: FP64 40^3 (250 tiles)
     // 0.041 against 0.054 ms, 48^3 (432) 0.064 against 0.059; FP32, two per
-    // CU, 48^3 0.038 against 0.053, 56^3 (686) 0.073 against 0.070
-    if (tiles_of<SmallTile>(G) <= SMAUG_CUS * fit) {
+    // CU, 48^3 0.038 against 0.053, 56^3 (686) 0.073 against 0.070.  It stages
+    // every box whatever the term mask says, in one round trip: that pays for
+    // the phases of v_f and b_f, which make a trip for each box otherwise
+    // (32^3 with hyperdiffusion off, RK4 step: 0.119 against 0.126 ms), and
+    // not for the fluxes, rho and e_int (16x12x12, single-stage step: fluxes
+    // only 0.0211 against 0.0168, with the rho terms 0.0220 against 0.0199)
+    const unsigned phases = SMAUG_T_ETERM | (G.hyper ? SMAUG_T_HMOM | SMAUG_T_HB : 0u);
+    if (tiles_of<SmallTile>(G) <= SMAUG_CUS * fit && (G.terms & phases)) {
       hipLaunchKernelGGL((k_rhs_small<SH>), dim3(tiles_of<SmallTile>(G)), dim3(SmallTile::NT), 0, st, G, A);
       return;
     }

@@ -94,7 +94,12 @@ inline int atomicOr(int* p, int v) {
   return o;
 }
 
-#define hipLaunchKernelGGL(K, G, B, S, ST, ...) emu::launch(dim3(G), dim3(B), [&]() { K(__VA_ARGS__); })
+// EMU_TRACE set: the launches by name on stderr
+#define hipLaunchKernelGGL(K, G, B, S, ST, ...)                    \
+  do {                                                             \
+    if (getenv("EMU_TRACE")) fprintf(stderr, "launch %s\n", #K);   \
+    emu::launch(dim3(G), dim3(B), [&]() { K(__VA_ARGS__); });      \
+  } while (0)
 
 hipError_t hipMalloc(void** p, size_t n);
 template <typename T>

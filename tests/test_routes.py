@@ -65,12 +65,16 @@ def libs(tmp_path_factory):
     return out
 
 
-def errors(lib, align, *case):
-    env = dict(os.environ, SMAUG_HIP_LIB=lib, EMU_ALIGN=align, OMP_NUM_THREADS="2", PYTHONPATH=ROOT)
+def child(lib, align, case, **env):
+    env = dict(os.environ, SMAUG_HIP_LIB=lib, EMU_ALIGN=align, OMP_NUM_THREADS="2", PYTHONPATH=ROOT, **env)
     p = subprocess.run([sys.executable, "-c", CHILD, json.dumps(case)], cwd=ROOT, env=env, capture_output=True,
                        text=True, timeout=300)
     assert p.returncode == 0, f"{case}: {p.stdout[-500:]}\n{p.stderr[-2000:]}"
-    return max(json.loads(p.stdout.strip().splitlines()[-1]))
+    return p
+
+
+def errors(lib, align, *case):
+    return max(json.loads(child(lib, align, case).stdout.strip().splitlines()[-1]))
 
 
 SIZES = [(12, 6, 6), (16, 8, 8), (17, 9, 12), (24, 7, 15), (32, 16, 8)]
@@ -92,6 +96,18 @@ def test_3d_boundaries_terms_and_other_grids(libs, route):
         assert errors(libs[route], "end", "strat", (17, 12, 10), 0, 0, 0, 4, terms) <= 1e-12, hex(terms)
     assert errors(libs[route], "end", "strat", (17, 12, 10), 1, 0, 1, 4, 0xFF) <= 1e-12
     assert errors(libs[route], "start", "strat", (17, 12, 10), 1, 1, 1, 4, 0xFF) <= 1e-5
+
+
+def test_small_grids_by_terms(libs):
+    """k_rhs_small stages every box of a tile; where the term mask leaves out
+    the phases of v_f and b_f, the tiled kernel runs, which stages less."""
+    flux, eterm, grav, hrho, he, hmom, hb, src = (1 << k for k in range(8))
+    for terms, kernel in ((0, "tiled"), (flux | grav | src, "tiled"), (flux | hrho | he, "tiled"), (flux | eterm, "small"),
+                          (hmom, "small"), (hb, "small"), (0xFF, "small")):
+        p = child(libs["small"], "end", ("strat", (12, 6, 6), 0, 0, 0, 4, terms), EMU_TRACE="1")
+        assert max(json.loads(p.stdout.strip().splitlines()[-1])) <= 1e-12, hex(terms)
+        ran = {k for k in ("tiled", "small", "wide", "general") if f"launch (k_rhs_{k}" in p.stderr}
+        assert ran == {kernel}, (hex(terms), ran)
 
 
 # 4 and 5 interior cells along an axis (the smallest the engine takes): a cell
