@@ -12,7 +12,8 @@ and kernels the GPU build compiles.
                                                        and vs the adjoint (dot products)
 
 case: s2r (2D stratified RK4), s2e (2D Euler), s3r (3D RK4), s3e (3D Euler,
-mixed only), ot (2D periodic).
+mixed only), ot (2D periodic), k2r, k3r (s2r, s3r on a grid that is no tensor
+product).
 """
 from __future__ import annotations
 
@@ -68,11 +69,13 @@ def make_case(name: str, terms: int = P.TERMS_ALL):
         rp.dt = 2e-3
         amap, il, nsteps = None, 9, 3
     else:
-        nd = 3 if name.startswith("s3") else 2
+        nd = 3 if name[1] == "3" else 2
         rkon = 0 if name.endswith("e") else 1
         rp, w, pos = strat_case(ni=(16, 12) if nd == 2 else (12, 8, 8), ndim=nd, rkon=rkon)
         amap = np.random.default_rng(3).uniform(150.0, 250.0, rp.ncells // rp.n[0])
         il, nsteps = (7, 3) if nd == 2 else (6, 2)
+    if name in ("k2r", "k3r"):  # s2r, s3r on positions that are no tensor product
+        pos = pos * (1.0 + 1e-3 * np.random.default_rng(5).random(pos.shape))
     rp.terms = terms
     return rp, w, pos, amap, il, nsteps
 

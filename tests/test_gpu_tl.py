@@ -438,6 +438,23 @@ def test_tl_mixed_precision_against_fp64(ni, i_line):
     assert et.max() > 0
 
 
+@pytest.mark.parametrize("ni,i_line", [((16, 12), 7), ((12, 8, 8), 6)])
+def test_tl_nonseparable_grid(ni, i_line):
+    """Positions that are no tensor product (the kernels of a general grid on
+    dual numbers): FP64 against the replayed differences, mixed precision
+    within 1e-5 of FP64."""
+    rp, w, pos = strat_tl_case(ni, len(ni), 1)
+    pos = pos * (1.0 + 1e-3 * np.random.default_rng(5).random(pos.shape))
+    tl_check(rp, w, pos, nsteps=3, i_line=i_line, per_field=False)
+    rng = np.random.default_rng(13)
+    inner = interior_mask(rp)
+    scale = np.sqrt((w[: P.npert(rp.ndim), inner] ** 2).mean(axis=1))
+    d = rng.standard_normal((scale.size, rp.ncells)) * scale[:, None] * inner[None, :]
+    (_, d64, w64, t64), (_, dm, wm, tm) = _tl_runs(rp, w, pos, d, 3, i_line)
+    assert _rel(wm, w64).max() <= 1e-5 and _rel(tm, t64).max() <= 1e-5
+    assert abs(dm - d64) <= 1e-5 * abs(d64), (dm, d64)
+
+
 def test_tl_mixed_c5_grid_192cubed():
     """The 3D adjoint configuration (192^3, FP32 shadows over an FP64 state):
     the derivative of the summed v_z^2 on the plane z ~ 4 Mm over 5 RK4 steps

@@ -99,7 +99,7 @@ def transposed(pair, tol=1e-10):
     return abs(got - want) <= tol * abs(want)
 
 
-@pytest.mark.parametrize("case", ["s2r", "s2e", "s3r", "ot", "tor", "spi", "bc:2d_fixed_asymm:0"])
+@pytest.mark.parametrize("case", ["s2r", "s2e", "s3r", "ot", "tor", "spi", "bc:2d_fixed_asymm:0", "k2r", "k3r"])
 def test_tangent_linear_matches_differences_and_adjoint(hostlib, case):
     """The tangent-linear run (smaug_tl_*): its values reproduce the oracle's
     loss, its directional derivatives of the line loss match the replayed
