@@ -91,7 +91,7 @@ __device__ inline void nu3_at(const Geo& G, const AdjArgs& A, const double* __re
   }
 }
 
-// (dF^d/du)^T Gf at one cell, added to lam.  F^d as in fluxes2:
+// (dF^d/du)^T Gf at one cell, added to lam.  F^d as in fluxes_of:
 //   F_rho  = v_d rho + rhob v_d                       (= m_d)
 //   F_m_f  = v_d m_f + [f=d] p_t - (b_f bb_d + bb_f b_d) - b_f b_d
 //   F_e    = v_d e + v_d p_t - b_d bb.v - bb_d b.v + v_d e_b - b_d b.v

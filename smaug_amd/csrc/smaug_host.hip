@@ -590,18 +590,8 @@ extern "C" int smaug_cfl(smaug_t* s, double* cmax_per_dim, double* dt) {
   if (cmax_per_dim)
     for (int d = 0; d < s->nd; d++) cmax_per_dim[d] = cm[d];
   if (dt) {
-    double v = dts[0];
-    if (s->p.moddton == 1) {  // from DT, then the CFL step if smaller (src/iosmaug.c:549-569)
-      double courantmax = 1.0e-12;
-      for (int d = 0; d < s->nd; d++) {
-        double t = cm[s->nd - 1] / s->p.dx[d];
-        if (t > courantmax) courantmax = t;
-      }
-      v = s->p.dt;
-      double dtt = s->p.courant / courantmax;
-      if (dtt > 1.0e-12 && dtt < s->p.dt) v = dtt;
-    }
-    *dt = v;
+    const double* dx = s->p.dx;
+    *dt = s->p.moddton == 1 ? cfl_dt(cm[s->nd - 1], s->nd, dx[0], dx[1], dx[2], s->p.courant, s->p.dt) : dts[0];
   }
   return check_flag(s);
 }

@@ -355,8 +355,10 @@ __device__ __forceinline__ void nu7(const T* Q, T dxk, T& nur, T& nul) {
 // Max ignores NaN as the reference's "if (v > max)" does.  A zero maximum
 // of the first differences (then the third ones are zero too) gives ratio 0
 // through the smallest normal numbers standing in for it: the quotient needs
-// no branch, and ratios are bounded by 6.  (Differences below 1e-300, or
-// 2e-38 in FP32, get a smaller ratio; their products are below 1e-300.)
+// no branch, and ratios are bounded by 6.  (Where all of an interface's first
+// differences are below 1e-300, or 2e-38 in FP32, the ratio comes out smaller
+// than it is: what such an interface diffuses, ratio times difference, is
+// below 6e-300, or 1.2e-37, times delx cmax chyp / delx^2 either way.)
 template <int NR, typename V>
 __device__ __forceinline__ void nu_ratios(const V* y, V* R) {
   const V tiny = sizeof(V) == 8 ? V(1e-300) : V(2e-38);
@@ -496,14 +498,6 @@ __device__ __forceinline__ void fluxes_of(const Geo& G, const CellState<ND, T>& 
 #pragma unroll
   for (int f = 0; f < ND; f++)
     F[fB(ND, f)] = (f == d) ? T(0) : vd * b[f] - (bd + bbd) * v[f] + bb[f] * vd;
-}
-
-template <int ND, typename SH>
-__device__ __forceinline__ void fluxes2(const Geo& G, const SH* __restrict__ w, const double* __restrict__ bg, long long cc,
-                               int d, double* F) {
-  CellState<ND> S;
-  load_cell<ND, SH>(G, w, bg, (unsigned)cc, S);
-  fluxes_of<ND>(G, S, d, F);
 }
 
 }  // namespace smaug
