@@ -21,9 +21,12 @@
 // The stencils work in the stencil precision SH: FP64 (the state itself),
 // or, in mixed precision, FP32 -- the shadows k_prim writes, FP32 LDS boxes
 // and FP32 arithmetic, which halves the LDS and most of the registers of a
-// workgroup and so raises the number resident per CU.  The own-cell values,
-// the background terms, the stage update (base + h*acc), the driver and the
-// RK combination are FP64 in both.
+// workgroup and so raises the number resident per CU.  A cell's own values in
+// the stencils come from the shadows too (rho_t: the FP32 rho plus the FP64
+// rho_b, rounded; m_f at the faces: rho_t v_f): with the FP64 rho instead a
+// step's errors against 64 bits agree to five digits (64^3 to 256^3).  The
+// background terms, gravity, the stage update (base + h*acc), the driver and
+// the RK combination are formed from FP64 values in both.
 //
 // What bounds it and how that shaped the code (MI355X):
 //  * a tile's phases are a chain of memory round trips and barriers, so time
@@ -38,10 +41,13 @@
 //    73 -> 48 us);
 //  * on grids of few tiles nothing hides a round trip: those keep every box
 //    in LDS at once (ALL: 6 barriers for 20, 48 -> 33 us per tile);
-//  * on large FP64 grids the traffic of the boxes counts: a tile of twice the
-//    cells re-reads a third less halo (k_rhs at 256^3: 4.60 ms before, 3.73
-//    with the small tile, 3.49 with the wide one; 15.1 GB fetched from beyond L2
-//    and 1.7 GB written, 4.8 TB/s of the 5.0 that a streaming pass reaches).
+//  * on large FP64 grids the boxes' traffic beyond L2 bounds it: 256^3 moves
+//    15.0 GB in and 1.7 GB out per launch, 4.7 TB/s of the 4.74 that a plain
+//    copy reaches.  Two cells per thread share addresses and the interface
+//    between them (22 % fewer VALU, 26 % fewer LDS and 55 % fewer vector memory
+//    instructions than the small tile, whose boxes are 25 % larger per cell
+//    but mostly found in L2: 15.3 GB): k_rhs at 256^3 4.61 ms before, 3.75
+//    with the small tile, 3.54 with the wide one.
 #include <math.h>
 
 #include <type_traits>
@@ -268,7 +274,7 @@ __device__ __forceinline__ void stage_rho_t(const Geo& G, const SH* __restrict__
 // The window of a thread's cells along direction D (0, 1, 2) of a q box:
 // the values at offsets -2..2 of each cell and nu_{i+1/2}, nu_{i-1/2} (sc =
 // delx * cmax * chyp).  The coefficient of an interface is a ratio of its own
-// (see nu_ratio), so two neighbours along dim 0 share the one between them.
+// (see nu_ratios), so two neighbours along dim 0 share the one between them.
 template <class TL, typename SH>
 struct Win {
   using V = typename ValT<SH>::T;
@@ -1402,7 +1408,7 @@ __global__ __launch_bounds__(SmallTile::NT, 1) void k_rhs_small(Geo G, RhsArgs A
 }
 
 // FP64 on large 3D tensor-product grids: two cells per thread, 8 x 8 x 8
-// tiles, three workgroups per CU (168 VGPRs, 53.5 KB of LDS).
+// tiles, three workgroups per CU (167 VGPRs, no scratch, 53.5 KB of LDS).
 __global__ __launch_bounds__(WideTile::NT, 3) void k_rhs_wide(Geo G, RhsArgs A) {
   using TL = WideTile;
   __shared__ __align__(16) double sm[Lay<TL>::SMEM];
